@@ -262,7 +262,7 @@ __device__ __forceinline__ void step_traj(const Fssh2Args* Ap, const Fssh2Args& 
     const double inv = 1.0 / (tn - L.tc);
     Interp2 P;
     P.dE0 = L.dEc; P.dE1 = (dEn - L.dEc) * inv; P.w0 = L.wc; P.w1 = (w - L.wc) * inv;
-    propagate2(P, L.s, L.t, L.tc, H.dt, H.nsub);
+    propagate2<R>(P, L.s, L.t, L.tc, H.dt, H.nsub);
     L.dEc = dEn; L.wc = w; L.tc = tn;
     L.t = tn;
     // A save time's values are those before the step's discrete callbacks (DiffEqBase's
@@ -379,7 +379,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void f
 }
 
 // FP64 (parity) path: three waves per SIMD without spilling.
-__global__ __launch_bounds__(256) void fssh2_persistent_f64(const Fssh2Args* __restrict__ Ap) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void fssh2_persistent_f64(const Fssh2Args* __restrict__ Ap) {
     persistent_body<1, double>(Ap);
 }
 

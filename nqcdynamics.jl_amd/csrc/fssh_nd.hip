@@ -348,7 +348,7 @@ __device__ __forceinline__ void nd_finish_step(const FsshNdArgs* Ap, const FsshN
     const double inv = 1.0 / (tn - L.tc);
     Interp2 P;
     P.dE0 = L.dEc; P.dE1 = (dEn - L.dEc) * inv; P.w0 = L.wc; P.w1 = (w - L.wc) * inv;
-    propagate2(P, L.s, L.t, L.tc, A.dt, A.nsub);
+    propagate2<R>(P, L.s, L.t, L.tc, A.dt, A.nsub);
     L.dEc = dEn; L.wc = w; L.tc = tn;
     L.t = tn;
     // the save precedes the hop callback (a save time holds the state before the step's callbacks)
@@ -458,7 +458,7 @@ __device__ __forceinline__ void nd_body(const FsshNdArgs* __restrict__ Ap, const
 }
 
 __global__ __launch_bounds__(256) void fssh_nd_f64(const FsshNdArgs* __restrict__ Ap) { nd_body<double, false>(Ap, nullptr); }
-__global__ __launch_bounds__(256) void fssh_nd_f32(const FsshNdArgs* __restrict__ Ap) { nd_body<float, false>(Ap, nullptr); }
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void fssh_nd_f32(const FsshNdArgs* __restrict__ Ap) { nd_body<float, false>(Ap, nullptr); }
 
 // Surrogate: the two packed members staged once into LDS, read by all eight wavefronts.
 constexpr int kMlpBlock = 512;

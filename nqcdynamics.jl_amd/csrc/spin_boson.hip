@@ -158,7 +158,13 @@ __device__ __forceinline__ void sb_body(const SbArgs* __restrict__ Ap) {
         const double inv = 1.0 / (tn - tc);
         Interp2 P;
         P.dE0 = dEc; P.dE1 = (dEn - dEc) * inv; P.w0 = wc; P.w1 = (w - wc) * inv;
-        propagate2(P, s, t, tc, A.dt, A.nsub);
+        {
+            Sig2 u = {0.5 * s.q, s.x, s.y};
+            const double s0 = t - tc;
+            propagate2_substeps(A.dt * fma(P.dE1, s0, P.dE0), (A.dt * A.dt) * P.dE1, (2.0 * A.dt) * fma(P.w1, s0, P.w0),
+                                (2.0 * A.dt * A.dt) * P.w1, A.nsub, u);
+            s.q = 2.0 * u.q; s.x = u.x; s.y = u.y;
+        }
         dEc = dEn; wc = w; tc = tn; t = tn;
         // the save precedes the hop callback (a save time holds the state before the step's callbacks)
         if (A.save_every > 0 && ((step + 1) % A.save_every) == 0) sb_save(Ap, tid, (step + 1) / A.save_every, method, st, tr, s, U);
