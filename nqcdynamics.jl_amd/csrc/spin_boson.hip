@@ -19,6 +19,8 @@
 namespace nqcd {
 
 constexpr int kBathModes = 100;  // instantiated bath size
+constexpr int kSbBlock = 64;     // one wavefront per workgroup
+constexpr int kSbAhead = 2;      // chunks of four modes whose coefficients are loaded together, one group ahead
 
 struct SbArgs {
     int64_t ntraj;
@@ -30,8 +32,8 @@ struct SbArgs {
     const double* w2;    // [NB] omega^2
     const double* c;     // [NB] coupling
     const double* invm;  // [NB] 1/m
-    const double* kd;    // [3][NB] half-kick coefficients dt/2 w^2/m, dt/2 c/m, and c (FP64)
-    const float* kf;     // [3][NB] the same in FP32
+    const double* kd;    // [NB/4][3][4] half-kick coefficients dt/2 w^2/m, dt/2 c/m, and c (FP64)
+    const float* kf;     // [NB/4][3][4] the same in FP32
     const double* r0;    // [NB][ntraj] sampled initial positions
     const double* v0;    // [NB][ntraj] sampled initial velocities
     double* r;           // [NB][ntraj]
@@ -75,30 +77,81 @@ __device__ __forceinline__ void sb_save(const SbArgs* Ap, int64_t tid, int slot,
     A.save_state[(int64_t)slot * n + tid] = st;
 }
 
+// The coefficient table through a constant-address-space pointer in scalar registers, made opaque where it is
+// used: its entries are scalar loads there, and go into the vector instructions as scalar operands.
+// Four modes make a chunk, so that a coefficient of a chunk is one four-wide load.
+template <typename R>
+using SbVec = R __attribute__((ext_vector_type(4)));
+template <typename R>
+using SbTab = __attribute__((address_space(4))) const SbVec<R>*;
+
 __device__ __forceinline__ const double* kick_table(const SbArgs& A, double) { return A.kd; }
 __device__ __forceinline__ const float* kick_table(const SbArgs& A, float) { return A.kf; }
 
-template <int NB, typename R>
-__device__ __forceinline__ void sb_body(const SbArgs* __restrict__ Ap) {
+template <typename R>
+__device__ __forceinline__ SbTab<R> sb_table(const SbArgs& A) {
+    return (SbTab<R>)uniform_sgpr((uint64_t)kick_table(A, (R)0));
+}
+
+template <typename R>
+__device__ __forceinline__ SbTab<R> sb_here(SbTab<R> p) {
+    asm volatile("" : "+s"(p));
+    return p;
+}
+
+// A step is two passes over the modes with the electronics between them.  Both half kicks that meet at a step
+// end see the same positions and the same force factor F (the acceleration of the step end stands, also after a
+// hop), so one pass applies them together: v = u - a is the velocity at the step end, whose projection on c the
+// coupling needs, and u' = 2 v - u the one after the next step's first half kick.
+//
+// The positions of the last NL modes stay in LDS ([chunk][lane], 16 bytes a lane and access), the rest and all
+// velocities in registers: with all 2 NB values in registers a wavefront took 352 registers, so the 1,563
+// wavefronts of 1e5 trajectories ran one to a SIMD in two rounds; with 48 of the FP32 positions in LDS two fit.
+// Bound by FP32 and FP64 issue (a step is about 600 FP32 instructions for the bath and 450 for the electronics).
+// 1e5 FSSH trajectories x 1000 steps: 23.7 -> 9.2 ms; before, the coefficients were vector loads through the
+// argument pointer, each waited for, 25 round trips to the cache per pass.
+template <int NB, int NL, typename R>
+__device__ __forceinline__ void sb_body(const SbArgs* __restrict__ Ap, SbVec<R>* lds) {
+    static_assert(NB % 4 == 0 && NL % 4 == 0 && NL < NB, "chunks of four modes");
+    constexpr int NC = NB / 4, NCR = (NB - NL) / 4;   // chunks, and those whose positions are in registers
     const SbArgs& A = *Ap;
     const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (tid >= A.ntraj) return;
+    if (tid >= A.ntraj) return;   // no barriers below: a lane reads only what it wrote
     const int method = A.method;
-    R x[NB], v[NB];
-    {
-        const SbArgs& B = *sb_opaque(Ap);
+    SbVec<R>* xl = lds + threadIdx.x;
+    R x[NB - NL], v[NB];
+    // the four positions of chunk q, from registers or LDS
+    auto load_x = [&](int q) -> SbVec<R> {
+        if (q < NCR) return SbVec<R>{x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]};
+        return xl[(q - NCR) * kSbBlock];
+    };
+    auto store_x = [&](int q, const SbVec<R>& xq) {
+        if (q < NCR) {
 #pragma unroll
-        for (int j = 0; j < NB; ++j) {
-            x[j] = (R)B.r0[(int64_t)j * B.ntraj + tid];
-            v[j] = (R)B.v0[(int64_t)j * B.ntraj + tid];
+            for (int k = 0; k < 4; ++k) x[4 * q + k] = xq[k];
+        } else {
+            xl[(q - NCR) * kSbBlock] = xq;
         }
-    }
-    // collective coordinate and the initial cache
+    };
+    const SbTab<R> K0 = sb_table<R>(A);
+    // collective coordinate X = sum c_j x_j of the initial positions
     R X = (R)0;
     {
-        const R* K = kick_table(*sb_opaque(Ap), (R)0);
+        const SbArgs& B = *sb_opaque(Ap);
+        const SbTab<R> K = sb_here<R>(K0);
 #pragma unroll
-        for (int j = 0; j < NB; ++j) X += K[2 * NB + j] * x[j];
+        for (int q = 0; q < NC; ++q) {
+            SbVec<R> xq;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                xq[k] = (R)B.r0[(int64_t)(4 * q + k) * B.ntraj + tid];
+                v[4 * q + k] = (R)B.v0[(int64_t)(4 * q + k) * B.ntraj + tid];
+            }
+            const SbVec<R> c = K[3 * q + 2];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) X += c[k] * xq[k];
+            store_x(q, xq);
+        }
     }
     double E0, E1, U[4];
     eigen2(A.eps + (double)X, A.Delta, -A.eps - (double)X, E0, E1, U, false);
@@ -124,108 +177,192 @@ __device__ __forceinline__ void sb_body(const SbArgs* __restrict__ Ap) {
     double dEc = 0.0, wc = 0.0, tc = 0.0, t = A.t0;
     int nh = 0;
     sb_save(Ap, tid, 0, method, st, tr, s, U);
-    const R dtR = (R)A.dt;
-    for (int step = 0; step < A.nsteps; ++step) {
-        // per-mode coefficients re-read every step (scalar loads) instead of being held in registers
-        const R* K = kick_table(*sb_opaque(Ap), (R)0);
-        const R Fr = (R)F;
-        R Xn = (R)0;
+    // the step loop's launch arguments in scalar registers
+    const int nsteps = (int)uniform_sgpr(A.nsteps), save_every = uniform_sgpr(A.save_every), nsub = uniform_sgpr(A.nsub);
+    const int rescaling = uniform_sgpr(A.rescaling);
+    const double dt = uniform_sgpr(A.dt), eps = uniform_sgpr(A.eps), Delta = uniform_sgpr(A.Delta);
+    const double S2 = uniform_sgpr(A.S2), cnorm = uniform_sgpr(A.cnorm);
+    const uint64_t key = uniform_sgpr(A.key);
+    const R dtR = (R)dt;
+    // v -= f (K x + C F), f = 1 (step_B!: v += dt/2 * k) or -1
+    auto half_kick = [&](R f, double Fd) {
+        const SbTab<R> K = sb_here<R>(K0);
+        const R Fr = (R)Fd;
 #pragma unroll
-        for (int j = 0; j < NB; ++j) {
-            v[j] = v[j] - (K[j] * x[j] + K[NB + j] * Fr);   // step_B!: v += dt/2 * k
-            x[j] = x[j] + dtR * v[j];                        // step_A!
-            Xn += K[2 * NB + j] * x[j];
+        for (int q = 0; q < NC; ++q) {
+            const SbVec<R> kx = K[3 * q], kf = K[3 * q + 1];
+            const SbVec<R> xq = load_x(q);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[4 * q + k] -= f * (kx[k] * xq[k] + kf[k] * Fr);
         }
-        eigen2(A.eps + (double)Xn, A.Delta, -A.eps - (double)Xn, E0, E1, U, true);  // update_cache!
+    };
+    if (nsteps > 0) half_kick((R)1, F);
+#pragma unroll 1
+    for (int step = 0; step < nsteps; ++step) {
+        R Xn = (R)0;
+        {
+            const SbTab<R> K = sb_here<R>(K0);
+            // the next group's coefficients and LDS positions are on their way while one is used
+            SbVec<R> c[2][kSbAhead], xa[2][kSbAhead];
+#pragma unroll
+            for (int i = 0; i < kSbAhead; ++i) c[0][i] = K[3 * i + 2];
+#pragma unroll
+            for (int q0 = 0; q0 < NC; q0 += kSbAhead) {
+                const int cur = (q0 / kSbAhead) & 1;
+#pragma unroll
+                for (int i = 0; i < kSbAhead; ++i) {
+                    const int q = q0 + kSbAhead + i;
+                    if (q < NC) c[cur ^ 1][i] = K[3 * q + 2];
+                    if (q < NC && q >= NCR) xa[cur ^ 1][i] = load_x(q);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < kSbAhead; ++i) {
+                    const int q = q0 + i;
+                    if (q >= NC) break;
+                    SbVec<R> xq = q < NCR ? load_x(q) : xa[cur][i];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        xq[k] = xq[k] + dtR * v[4 * q + k];          // step_A!
+                        Xn += c[cur][i][k] * xq[k];
+                    }
+                    store_x(q, xq);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        eigen2(eps + (double)Xn, Delta, -eps - (double)Xn, E0, E1, U, true);  // update_cache!
         rotate_sz(U, g00, g11, g01);
         {
             const double aa = 0.5 * (tr + s.q), bb = 0.5 * (tr - s.q);
             F = (method == 0) ? ((st == 0) ? g00 : g11) : (g00 * aa + g11 * bb + 2.0 * g01 * s.x);
         }
-        const R* K2 = kick_table(*sb_opaque(Ap), (R)0);
-        const R Fn = (R)F;
         R Vc = (R)0;
+        {
+            const SbTab<R> K = sb_here<R>(K0);
+            const R Fn = (R)F;
+            SbVec<R> c[2][kSbAhead][3], xa[2][kSbAhead];
 #pragma unroll
-        for (int j = 0; j < NB; ++j) {
-            v[j] = v[j] - (K2[j] * x[j] + K2[NB + j] * Fn);  // step_B!
-            Vc += K2[2 * NB + j] * v[j];
+            for (int i = 0; i < 3 * kSbAhead; ++i) c[0][i / 3][i % 3] = K[i];
+#pragma unroll
+            for (int q0 = 0; q0 < NC; q0 += kSbAhead) {
+                const int cur = (q0 / kSbAhead) & 1;
+#pragma unroll
+                for (int i = 0; i < 3 * kSbAhead; ++i)
+                    if (q0 + kSbAhead + i / 3 < NC) c[cur ^ 1][i / 3][i % 3] = K[3 * (q0 + kSbAhead) + i];
+#pragma unroll
+                for (int i = 0; i < kSbAhead; ++i)
+                    if (q0 + kSbAhead + i < NC && q0 + kSbAhead + i >= NCR) xa[cur ^ 1][i] = load_x(q0 + kSbAhead + i);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < kSbAhead; ++i) {
+                    const int q = q0 + i;
+                    if (q >= NC) break;
+                    const SbVec<R> xq = q < NCR ? load_x(q) : xa[cur][i];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {                    // step_B! twice
+                        const R vn = v[4 * q + k] - c[cur][i][0][k] * xq[k] - c[cur][i][1][k] * Fn;
+                        Vc += c[cur][i][2][k] * vn;
+                        v[4 * q + k] = (R)2 * vn - v[4 * q + k];
+                        asm volatile("" : "+v"(v[4 * q + k]));   // formed here: left to be sunk, vn and the old v both live on
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
         const double gap = E1 - E0;
         const double d01c = g01 / gap;               // d_j[0][1] = c_j * d01c
         const double w = d01c * (double)Vc;
-        const double tn = t + A.dt;
+        const double tn = t + dt;
         const double dEn = E0 - E1;
         const double inv = 1.0 / (tn - tc);
         Interp2 P;
         P.dE0 = dEc; P.dE1 = (dEn - dEc) * inv; P.w0 = wc; P.w1 = (w - wc) * inv;
-        {
-            Sig2 u = {0.5 * s.q, s.x, s.y};
-            const double s0 = t - tc;
-            propagate2_substeps(A.dt * fma(P.dE1, s0, P.dE0), (A.dt * A.dt) * P.dE1, (2.0 * A.dt) * fma(P.w1, s0, P.w0),
-                                (2.0 * A.dt * A.dt) * P.w1, A.nsub, u);
-            s.q = 2.0 * u.q; s.x = u.x; s.y = u.y;
-        }
+        // 100 modes carry a step's difference on: held two orders tighter beside FP64 nuclei
+        propagate2<R>(P, s, t, tc, dt, nsub, 1e-14);
         dEc = dEn; wc = w; tc = tn; t = tn;
         // the save precedes the hop callback (a save time holds the state before the step's callbacks)
-        if (A.save_every > 0 && ((step + 1) % A.save_every) == 0) sb_save(Ap, tid, (step + 1) / A.save_every, method, st, tr, s, U);
+        if (save_every > 0 && ((step + 1) % save_every) == 0) sb_save(Ap, tid, (step + 1) / save_every, method, st, tr, s, U);
         if (method == 0) {
             const double sss = 0.5 * (tr + ((st == 0) ? s.q : -s.q));
             const double ratio = s.x / sss;
             const double dsm = (st == 0) ? d01c : -d01c;
-            double p = 2.0 * (double)Vc * ratio * dsm * A.dt;
+            double p = 2.0 * (double)Vc * ratio * dsm * dt;
+            // the velocities' change of an accepted or reflected hop, v_j -= (s1 / m_j + s2) c_j
+            double s1 = 0.0, s2 = 0.0;
             if (p > 0.0) {
                 p = fmin(p, 1.0);
-                const double rnd = philox_uniform((uint64_t)tid, (uint32_t)step, STREAM_HOP, A.key);
+                const double rnd = philox_uniform((uint64_t)tid, (uint32_t)step, STREAM_HOP, key);
                 if (p > rnd) {
                     // rescale along d_j = c_j * dms (coupling[new, old]); surface_hopping.jl:64-99
                     const double dms = -dsm;
                     const double dE = (st == 0) ? gap : -gap;
                     bool accept = true;
-                    if (A.rescaling != 2) {
-                        const double aq = 0.5 * dms * dms * A.S2;
+                    if (rescaling != 2) {
+                        const double aq = 0.5 * dms * dms * S2;
                         const double bq = dms * (double)Vc;
                         const double disc = bq * bq - 4.0 * aq * dE;
                         if (disc < 0.0) {
                             accept = false;
-                            if (A.rescaling == 1) {
-                                const SbArgs& C = *sb_opaque(Ap);
-                                const double nrm = fabs(dms) * A.cnorm;
-                                const double gam = bq / nrm;
-#pragma unroll
-                                for (int j = 0; j < NB; ++j)
-                                    v[j] = (R)((double)v[j] - 2.0 * gam * (dms * C.c[j] / nrm));
+                            if (rescaling == 1) {
+                                const double nrm = fabs(dms) * cnorm;
+                                s2 = 2.0 * (bq / nrm) * (dms / nrm);
                             }
                         } else {
-                            const SbArgs& C = *sb_opaque(Ap);
                             const double root = sqrt(disc);
                             const double gam = (bq < 0.0) ? (bq + root) / (2.0 * aq) : (bq - root) / (2.0 * aq);
-#pragma unroll
-                            for (int j = 0; j < NB; ++j) v[j] = (R)((double)v[j] - gam * dms * C.c[j] * C.invm[j]);
+                            s1 = gam * dms;
                         }
                     }
                     if (accept) { st = 1 - st; ++nh; }
                 }
             }
+            // one pass for the wavefront (a zero change leaves the other lanes' velocities as they are), so the
+            // velocities are not copied around a divergent region every step
+            if (__ballot(s1 != 0.0 || s2 != 0.0) != 0) {
+                const SbTab<double> cm = (SbTab<double>)uniform_sgpr((uint64_t)sb_opaque(Ap)->c);
+                const SbTab<double> im = (SbTab<double>)uniform_sgpr((uint64_t)sb_opaque(Ap)->invm);
+#pragma unroll
+                for (int q = 0; q < NC; ++q) {
+                    const SbVec<double> cq = cm[q], iq = im[q];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) v[4 * q + k] = (R)((double)v[4 * q + k] - (s1 * iq[k] + s2) * cq[k]);
+                    __builtin_amdgcn_sched_barrier(0);   // chunk by chunk: converted all at once they spill
+                }
+            }
         }
     }
+    if (nsteps > 0) half_kick((R)-1, F);   // the next step's first half kick taken back
     const SbArgs& B = *sb_opaque(Ap);
     const int64_t n = B.ntraj;
 #pragma unroll
-    for (int j = 0; j < NB; ++j) {
-        B.r[(int64_t)j * n + tid] = (double)x[j];
-        B.v[(int64_t)j * n + tid] = (double)v[j];
+    for (int q = 0; q < NC; ++q) {
+        const SbVec<R> xq = load_x(q);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            B.r[(int64_t)(4 * q + k) * n + tid] = (double)xq[k];
+            B.v[(int64_t)(4 * q + k) * n + tid] = (double)v[4 * q + k];
+        }
     }
     B.sig[tid] = 0.5 * (tr + s.q);
     B.sig[n + tid] = 0.5 * (tr - s.q);
     B.sig[2 * n + tid] = s.x;
     B.sig[3 * n + tid] = s.y;
     B.state[tid] = st;
-    B.steps[tid] = (int32_t)A.nsteps;
+    B.steps[tid] = (int32_t)nsteps;
     B.nhops[tid] = nh;
 }
 
-__global__ __launch_bounds__(64) void sb_kernel_f32(const SbArgs* __restrict__ Ap) { sb_body<kBathModes, float>(Ap); }
-__global__ __launch_bounds__(64) void sb_kernel_f64(const SbArgs* __restrict__ Ap) { sb_body<kBathModes, double>(Ap); }
+constexpr int kSbLds32 = 48, kSbLds64 = 40;   // modes whose positions are in LDS (12 KB, 20 KB a wavefront)
+__global__ __launch_bounds__(kSbBlock) __attribute__((amdgpu_waves_per_eu(2)))
+void sb_kernel_f32(const SbArgs* __restrict__ Ap) {
+    __shared__ SbVec<float> lds[kSbLds32 / 4 * kSbBlock];
+    sb_body<kBathModes, kSbLds32, float>(Ap, lds);
+}
+__global__ __launch_bounds__(kSbBlock) void sb_kernel_f64(const SbArgs* __restrict__ Ap) {
+    __shared__ SbVec<double> lds[kSbLds64 / 4 * kSbBlock];
+    sb_body<kBathModes, kSbLds64, double>(Ap, lds);
+}
 
 // ---------------------------------------------------------------------------
 // Host side.
@@ -249,10 +386,11 @@ int32_t sb_sample_initial(nqcd_handle_t* h, const nqcd_sampler_desc* S, uint64_t
     const double hdt = 0.5 * h->prob.dt;
     std::vector<float> tabf(3 * nb);
     for (int j = 0; j < nb; ++j) {
-        tab[7 * nb + j] = hdt * tab[j] * tab[2 * nb + j];
-        tab[8 * nb + j] = hdt * tab[nb + j] * tab[2 * nb + j];
-        tab[9 * nb + j] = tab[nb + j];
-        for (int k = 0; k < 3; ++k) tabf[k * nb + j] = (float)tab[(7 + k) * nb + j];
+        double* t4 = tab.data() + 7 * nb + 12 * (j / 4) + j % 4;   // chunks of four modes: kick, force and c
+        t4[0] = hdt * tab[j] * tab[2 * nb + j];
+        t4[4] = hdt * tab[nb + j] * tab[2 * nb + j];
+        t4[8] = tab[nb + j];
+        for (int k = 0; k < 3; ++k) tabf[12 * (j / 4) + 4 * k + j % 4] = (float)t4[4 * k];
     }
     HIPCHK(h, hipMemcpy(h->bath.p, tab.data(), sizeof(double) * 10 * nb, hipMemcpyHostToDevice));
     HIPCHK(h, hipMemcpy(h->bath.as<char>() + sizeof(double) * 10 * nb, tabf.data(), sizeof(float) * 3 * nb,
@@ -316,7 +454,7 @@ int32_t sb_run(nqcd_handle_t* h, double t0, int64_t nsteps, const nqcd_term_desc
     A.save_state = h->save_state.as<int32_t>();
     HIPCHK(h, h->args_dev.ensure(sizeof(SbArgs)));
     HIPCHK(h, hipMemcpyAsync(h->args_dev.p, &A, sizeof(SbArgs), hipMemcpyHostToDevice, h->stream));
-    const int block = 64;
+    const int block = kSbBlock;
     const int grid = (int)((n + block - 1) / block);
     HIPCHK(h, hipEventRecord(h->ev0, h->stream));
     if (h->prob.precision == NQCD_PREC_FP64)
