@@ -14,7 +14,7 @@ constexpr int kNsMaxStates = 8;
 struct FsshNArgs {
     int64_t ntraj;
     int32_t method, rescaling, nsub, save_every;
-    int32_t nsave, term_kind, init_diabatic, pad;
+    int32_t nsave, term_kind, init_diabatic, ntab;   // ntab: doubles in mtab, staged in LDS
     int32_t slot_n[kMaxModels];     // states of each model slot
     int32_t slot_tab[kMaxModels];   // offset of a MORSE_N slot's table in mtab, -1 for closed-form models
     double term_value, dt, t0, inv_mass;
@@ -52,8 +52,8 @@ int32_t ns_load_initial(nqcd_handle_t* h, int64_t ntraj, const double* r, const 
 int32_t ns_sample_initial(nqcd_handle_t* h, const nqcd_sampler_desc* S, uint64_t seed);
 int32_t ns_run(nqcd_handle_t* h, double t0, int64_t nsteps, const nqcd_term_desc* term, uint64_t key);
 int32_t ns_download(nqcd_handle_t* h, int32_t field, void* out, int64_t bytes);
-// Launch and occupancy of the five- to eight-state kernels (fssh_n8.hip).
-hipError_t ns_launch_hi(int NM, int precision, int grid, int block, hipStream_t s, const FsshNArgs* Adev);
-hipError_t ns_occupancy_hi(int NM, int precision, int block, int* bpc);
+// The five- to eight-state kernels (fssh_n8.hip).
+using NsKernelPtr = void (*)(const FsshNArgs*);
+NsKernelPtr ns_kernel_hi(int NM, int precision, bool five_substeps);
 
 }  // namespace nqcd

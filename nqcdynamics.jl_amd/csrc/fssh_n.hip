@@ -45,32 +45,13 @@ __global__ void ns_queue_reset(unsigned long long* q) { *q = 0ull; }
 // ---------------------------------------------------------------------------
 int ns_kernel_states(int n) { return n < 2 ? 2 : n; }
 
-static hipError_t ns_launch(int NM, int precision, int grid, int block, hipStream_t s, const FsshNArgs* Adev) {
-    if (NM > 4) return ns_launch_hi(NM, precision, grid, block, s, Adev);
-#define NQCD_CASE(X)                                                                                         \
-    case X:                                                                                                  \
-        if (precision == 0) hipLaunchKernelGGL(fssh_n_f64_##X, dim3(grid), dim3(block), 0, s, Adev);         \
-        else hipLaunchKernelGGL(fssh_n_f32_##X, dim3(grid), dim3(block), 0, s, Adev);                        \
-        break;
+static NsKernelPtr ns_kernel(int NM, int precision, bool five) {
     switch (NM) {
-        NQCD_CASE(2) NQCD_CASE(3) NQCD_CASE(4)
-    default: return hipErrorInvalidValue;
+    case 2: return NQCD_NS_PICK(2, precision, five);
+    case 3: return NQCD_NS_PICK(3, precision, five);
+    case 4: return NQCD_NS_PICK(4, precision, five);
+    default: return ns_kernel_hi(NM, precision, five);
     }
-#undef NQCD_CASE
-    return hipGetLastError();
-}
-
-static hipError_t ns_occupancy(int NM, int precision, int block, int* bpc) {
-    if (NM > 4) return ns_occupancy_hi(NM, precision, block, bpc);
-#define NQCD_CASE(X)                                                                                         \
-    case X:                                                                                                  \
-        return precision == 0 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(bpc, fssh_n_f64_##X, block, 0)  \
-                              : hipOccupancyMaxActiveBlocksPerMultiprocessor(bpc, fssh_n_f32_##X, block, 0);
-    switch (NM) {
-        NQCD_CASE(2) NQCD_CASE(3) NQCD_CASE(4)
-    default: return hipErrorInvalidValue;
-    }
-#undef NQCD_CASE
 }
 
 bool ns_is_problem(const nqcd_handle_t* h) {
@@ -267,9 +248,13 @@ int32_t ns_run(nqcd_handle_t* h, double t0, int64_t nsteps, const nqcd_term_desc
     A.save_pop_ad = h->save_ad.as<double>(); A.save_pop_di = h->save_di.as<double>();
     A.save_state = h->save_state.as<int32_t>();
     A.queue = h->queue.as<unsigned long long>();
+    A.ntab = (int32_t)tab.size();
+    const size_t lds = sizeof(double) * tab.size();   // at most 4 slots of 116 doubles
+    const NsKernelPtr kernel = ns_kernel(NM, h->prob.precision, A.nsub == 5);
+    if (!kernel) return fail(h, NQCD_ERR_UNSUPPORTED, "n-state kernels exist for 2 to 8 states");
     const int block = 256;
     int bpc = 0;
-    HIPCHK(h, ns_occupancy(NM, h->prob.precision, block, &bpc));
+    HIPCHK(h, hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, (const void*)kernel, block, lds));
     if (bpc < 1) bpc = 1;
     const int64_t lanes = (int64_t)bpc * h->cu_count * block;
     const int64_t grid = std::max<int64_t>(1, std::min<int64_t>((nt + block - 1) / block, lanes / block));
@@ -277,7 +262,8 @@ int32_t ns_run(nqcd_handle_t* h, double t0, int64_t nsteps, const nqcd_term_desc
     HIPCHK(h, hipMemcpyAsync(h->args_dev.p, &A, sizeof(FsshNArgs), hipMemcpyHostToDevice, h->stream));
     HIPCHK(h, hipEventRecord(h->ev0, h->stream));
     hipLaunchKernelGGL(ns_queue_reset, dim3(1), dim3(1), 0, h->stream, A.queue);
-    HIPCHK(h, ns_launch(NM, h->prob.precision, (int)grid, block, h->stream, h->args_dev.as<const FsshNArgs>()));
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(block), lds, h->stream, h->args_dev.as<const FsshNArgs>());
+    HIPCHK(h, hipGetLastError());
     HIPCHK(h, hipEventRecord(h->ev1, h->stream));
     h->stats.block = block;
     h->stats.grid = (int)grid;

@@ -9,30 +9,14 @@ NQCD_NS_KERNELS(6)
 NQCD_NS_KERNELS(7)
 NQCD_NS_KERNELS(8)
 
-hipError_t ns_launch_hi(int NM, int precision, int grid, int block, hipStream_t s, const FsshNArgs* Adev) {
-#define NQCD_CASE(X)                                                                                         \
-    case X:                                                                                                  \
-        if (precision == 0) hipLaunchKernelGGL(fssh_n_f64_##X, dim3(grid), dim3(block), 0, s, Adev);         \
-        else hipLaunchKernelGGL(fssh_n_f32_##X, dim3(grid), dim3(block), 0, s, Adev);                        \
-        break;
+NsKernelPtr ns_kernel_hi(int NM, int precision, bool five) {
     switch (NM) {
-        NQCD_CASE(5) NQCD_CASE(6) NQCD_CASE(7) NQCD_CASE(8)
-    default: return hipErrorInvalidValue;
+    case 5: return NQCD_NS_PICK(5, precision, five);
+    case 6: return NQCD_NS_PICK(6, precision, five);
+    case 7: return NQCD_NS_PICK(7, precision, five);
+    case 8: return NQCD_NS_PICK(8, precision, five);
+    default: return nullptr;
     }
-#undef NQCD_CASE
-    return hipGetLastError();
-}
-
-hipError_t ns_occupancy_hi(int NM, int precision, int block, int* bpc) {
-#define NQCD_CASE(X)                                                                                         \
-    case X:                                                                                                  \
-        return precision == 0 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(bpc, fssh_n_f64_##X, block, 0)  \
-                              : hipOccupancyMaxActiveBlocksPerMultiprocessor(bpc, fssh_n_f32_##X, block, 0);
-    switch (NM) {
-        NQCD_CASE(5) NQCD_CASE(6) NQCD_CASE(7) NQCD_CASE(8)
-    default: return hipErrorInvalidValue;
-    }
-#undef NQCD_CASE
 }
 
 }  // namespace nqcd

@@ -25,7 +25,7 @@ struct LaneN {
     double U[NM * NM];                                     // eigenvectors, row-major, column j = state j
     double Ec[NM], Wc[NP > 0 ? NP : 1];                    // electronic buffer at the step start
     double tc, t;
-    const double* tab;                                     // MORSE_N table of the trajectory's model, or null
+    const double* tab;                                     // MORSE_N table of the trajectory's model (LDS or global), or null
     ModelRegs m;
     int64_t tid;
     int32_t n, st, nh, step;
@@ -135,21 +135,23 @@ __device__ __forceinline__ void ns_eigen(int n, const double vd[NM], const doubl
 #pragma unroll
             for (int q = p + 1; q < NM; ++q) {
                 const double apq = A[p * NM + q];
-                if (q < n && apq != 0.0) {
-                    const double theta = (A[q * NM + q] - A[p * NM + p]) / (2.0 * apq);
-                    const double t = (theta >= 0.0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0));
-                    const double c = 1.0 / sqrt(t * t + 1.0), s = t * c;
+                // t = tan of the rotation angle, the smaller root: 2 a_pq sgn(h) / (|h| + sqrt(h^2 + 4 a_pq^2)),
+                // h = a_qq - a_pp.  Square roots and reciprocals by the hardware estimate and Newton steps: a
+                // rotation's last bit only moves what the next sweep removes.
+                const double h = A[q * NM + q] - A[p * NM + p], t2 = 2.0 * apq, r2 = fma(h, h, t2 * t2);
+                if (q < n && apq != 0.0 && r2 > 0.0) {
+                    const double t = (h >= 0.0 ? t2 : -t2) * nr_rcp(fabs(h) + r2 * nr_rsq(r2));
+                    const double c = nr_rsq(fma(t, t, 1.0)), s = t * c;
+                    A[p * NM + p] -= t * apq;   // A <- J^T A J, the pair annihilated
+                    A[q * NM + q] += t * apq;
+                    A[p * NM + q] = 0.0;
+                    A[q * NM + p] = 0.0;
 #pragma unroll
-                    for (int k = 0; k < NM; ++k) {  // A <- A J (columns p, q)
+                    for (int k = 0; k < NM; ++k) {
+                        if (k == p || k == q) continue;
                         const double akp = A[k * NM + p], akq = A[k * NM + q];
-                        A[k * NM + p] = c * akp - s * akq;
-                        A[k * NM + q] = s * akp + c * akq;
-                    }
-#pragma unroll
-                    for (int k = 0; k < NM; ++k) {  // A <- J^T A (rows p, q)
-                        const double apk = A[p * NM + k], aqk = A[q * NM + k];
-                        A[p * NM + k] = c * apk - s * aqk;
-                        A[q * NM + k] = s * apk + c * aqk;
+                        A[k * NM + p] = A[p * NM + k] = c * akp - s * akq;
+                        A[k * NM + q] = A[q * NM + k] = s * akp + c * akq;
                     }
 #pragma unroll
                     for (int k = 0; k < NM; ++k) {
@@ -253,37 +255,99 @@ __device__ __forceinline__ void ns_rotate(const double U[NM * NM], const double 
         }
 }
 
-// Right-hand side of the density equation, K = f(a, x, y) at energies e and couplings w (upper).
-template <int NM>
+// Right-hand side of the density equation at energies e and couplings W = w (upper, antisymmetric), written out
+// for the real diagonal a and the upper elements x + i y of sigma:
+//   a_i'  = -2 sum_k W_ik x_ki
+//   x_ij' = (e_i - e_j) y_ij - W_ij (a_j - a_i) - sum_{k != i, j} (W_ik x_kj + W_jk x_ki)
+//   y_ij' = -(e_i - e_j) x_ij - sum_{k != i, j} (W_ik y_kj - W_jk y_ki)
+// ADD: added to ka, kx, ky (every product is then a fused multiply-add), else stored there.
+template <int NM, bool ADD>
 __device__ __forceinline__ void ns_rhs(const double e[NM], const double w[], const double a[NM], const double x[],
                                        const double y[], double ka[NM], double kx[], double ky[]) {
-    auto W = [&](int i, int k) -> double { return i == k ? 0.0 : (i < k ? w[pidx<NM>(i, k)] : -w[pidx<NM>(k, i)]); };
-    auto X = [&](int k, int j) -> double { return k == j ? a[k] : (k < j ? x[pidx<NM>(k, j)] : x[pidx<NM>(j, k)]); };
-    auto Y = [&](int k, int j) -> double { return k == j ? 0.0 : (k < j ? y[pidx<NM>(k, j)] : -y[pidx<NM>(j, k)]); };
-    double M[NM * NM], N[NM * NM];
+    auto W = [&](int i, int k) -> double { return i < k ? w[pidx<NM>(i, k)] : -w[pidx<NM>(k, i)]; };
+    auto X = [&](int k, int j) -> double { return k < j ? x[pidx<NM>(k, j)] : x[pidx<NM>(j, k)]; };
+    auto Y = [&](int k, int j) -> double { return k < j ? y[pidx<NM>(k, j)] : -y[pidx<NM>(j, k)]; };
 #pragma unroll
-    for (int i = 0; i < NM; ++i)
+    for (int i = 0; i < NM; ++i) {
+        double s = 0.0;
 #pragma unroll
-        for (int j = 0; j < NM; ++j) {
-            double sm = 0.0, sn = 0.0;
-#pragma unroll
-            for (int k = 0; k < NM; ++k) {
-                if (k != i) { sm += W(i, k) * X(k, j); sn += W(i, k) * Y(k, j); }
-            }
-            M[i * NM + j] = sm;
-            N[i * NM + j] = sn;
-        }
-#pragma unroll
-    for (int i = 0; i < NM; ++i) ka[i] = -2.0 * M[i * NM + i];
+        for (int k = 0; k < NM; ++k)
+            if (k != i) s = fma(W(i, k), X(i, k), s);
+        ka[i] = ADD ? fma(-2.0, s, ka[i]) : -2.0 * s;
+    }
 #pragma unroll
     for (int i = 0; i < NM; ++i)
 #pragma unroll
         for (int j = i + 1; j < NM; ++j) {
             const int p = pidx<NM>(i, j);
             const double de = e[i] - e[j];
-            kx[p] = de * y[p] - (M[i * NM + j] + M[j * NM + i]);
-            ky[p] = -de * x[p] - (N[i * NM + j] - N[j * NM + i]);
+            double fx = ADD ? kx[p] : 0.0, fy = ADD ? ky[p] : 0.0;
+#pragma unroll
+            for (int k = 0; k < NM; ++k) {
+                if (k == i || k == j) continue;
+                fx = fma(-W(i, k), X(k, j), fma(-W(j, k), X(k, i), fx));
+                fy = fma(-W(i, k), Y(k, j), fma(W(j, k), Y(k, i), fy));
+            }
+            kx[p] = fma(de, y[p], fma(-w[p], a[j] - a[i], fx));
+            ky[p] = fma(-de, x[p], fy);
         }
+}
+
+// 1 / k!, read with scalar loads by the rolled series
+__constant__ double kInvFactorial[21] = {1.0, 1.0, 1.0 / 2.0, 1.0 / 6.0, 1.0 / 24.0, 1.0 / 120.0, 1.0 / 720.0, 1.0 / 5040.0,
+    1.0 / 40320.0, 1.0 / 362880.0, 1.0 / 3628800.0, 1.0 / 39916800.0, 1.0 / 479001600.0, 1.0 / 6227020800.0,
+    1.0 / 87178291200.0, 1.0 / 1307674368000.0, 1.0 / 20922789888000.0, 1.0 / 355687428096000.0, 1.0 / 6402373705728000.0,
+    1.0 / 121645100408832000.0, 1.0 / 2432902008176640000.0};
+
+// The density over a nuclear step as one power series (series_step2 in nqcd_device.h, for the n-state equation):
+// over the step the energies and couplings are e + e1 s, w + w1 s for s in [0, 1] (times dt), so the derivatives
+// obey u^(k+1) = f(e, w; u^(k)) + k f(e1, w1; u^(k-1)), two right-hand sides an order in place of the 31 and the
+// stage sums of five Tsit5 sub-steps.  Orders by z2 = |A0|^2 + 4 |A1| as there, with
+// |A| <= spread of the energies + 2 sum |w|.  Bound by FP64 issue; without the stages of five sub-steps the
+// three-state FP32 kernel needs 214 registers instead of 256 and runs two wavefronts a SIMD (1e5 three-state Morse
+// trajectories x 1000 steps, with the cheaper Jacobi rotations and the tables in LDS: 20.8 -> 8.9 ms).
+__device__ __forceinline__ int ns_series_orders(double z2) {
+    return z2 > 0.0041 ? (z2 > 0.022 ? (z2 > 0.075 ? (z2 > 0.19 ? (z2 > 0.35 ? (z2 > 0.65 ? 20 : 18) : 16) : 14) : 12) : 10) : 8;
+}
+
+template <int NM>
+__device__ __forceinline__ double ns_norm(int n, const double e[NM], const double w[]) {
+    constexpr int NP = NM * (NM - 1) / 2;
+    double lo = e[0], hi = e[0], sw = 0.0;
+#pragma unroll
+    for (int i = 1; i < NM; ++i)
+        if (i < n) { lo = fmin(lo, e[i]); hi = fmax(hi, e[i]); }
+#pragma unroll
+    for (int p = 0; p < NP; ++p) sw += fabs(w[p]);
+    return fma(2.0, sw, hi - lo);
+}
+
+template <int NM>
+__device__ __forceinline__ void ns_series(const double e[NM], const double w[], const double e1[NM], const double w1[],
+                                          int orders, double a[NM], double x[], double y[]) {
+    constexpr int NP = NM * (NM - 1) / 2;
+    constexpr int NQ = NP > 0 ? NP : 1;
+    double ka[NM], kx[NQ], ky[NQ], pa[NM], px[NQ], py[NQ];   // u^(k) and u^(k-1)
+    double ek[NM], wk[NQ];                                     // k times the slopes
+#pragma unroll
+    for (int i = 0; i < NM; ++i) { ka[i] = a[i]; pa[i] = 0.0; ek[i] = 0.0; }
+#pragma unroll
+    for (int p = 0; p < NP; ++p) { kx[p] = x[p]; ky[p] = y[p]; px[p] = 0.0; py[p] = 0.0; wk[p] = 0.0; }
+#pragma unroll 1
+    for (int k = 1; k <= orders; ++k) {
+        const double rf = kInvFactorial[k];
+        double fa[NM], fx[NQ], fy[NQ];
+        ns_rhs<NM, false>(ek, wk, pa, px, py, fa, fx, fy);
+        ns_rhs<NM, true>(e, w, ka, kx, ky, fa, fx, fy);
+#pragma unroll
+        for (int i = 0; i < NM; ++i) { pa[i] = ka[i]; ka[i] = fa[i]; a[i] = fma(fa[i], rf, a[i]); ek[i] += e1[i]; }
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            px[p] = kx[p]; kx[p] = fx[p]; x[p] = fma(fx[p], rf, x[p]);
+            py[p] = ky[p]; ky[p] = fy[p]; y[p] = fma(fy[p], rf, y[p]);
+            wk[p] += w1[p];
+        }
+    }
 }
 
 // One Tsit5 step of size h from tau (electronic_dynamics.jl:104-130 integrated by Tsit5, the stage
@@ -343,7 +407,7 @@ __device__ __forceinline__ void ns_tsit5(const NsInterp<NM>& I, double tau, doub
             ty[p] = (st == 0) ? y[p] : y[p] + h * sy;
         }
         ns_params<NM>(I, tau + cs[st] * h, e, w);
-        ns_rhs<NM>(e, w, ta, tx, ty, ka[st], kx[st], ky[st]);
+        ns_rhs<NM, false>(e, w, ta, tx, ty, ka[st], kx[st], ky[st]);
     }
     const double b[6] = {a71, a72, a73, a74, a75, a76};
 #pragma unroll
@@ -363,8 +427,9 @@ __device__ __forceinline__ void ns_tsit5(const NsInterp<NM>& I, double tau, doub
     }
 }
 
-template <int NM, typename R>
-__device__ __forceinline__ void ns_accel(const FsshNArgs& A, LaneN<NM, R>& L, const double Gd[NM], const double Go[],
+// A: FsshNArgs, or NsHot (its fields in scalar registers)
+template <int NM, typename R, class AT>
+__device__ __forceinline__ void ns_accel(const AT& A, LaneN<NM, R>& L, const double Gd[NM], const double Go[],
                                          const double* aa, const double* xx) {
     constexpr int NP = LaneN<NM, R>::NP;
     double f;
@@ -412,14 +477,14 @@ __device__ __forceinline__ void ns_save(const FsshNArgs* Ap, const LaneN<NM, R>&
 }
 
 template <int NM, typename R>
-__device__ __forceinline__ void ns_load(const FsshNArgs* Ap, LaneN<NM, R>& L, int64_t tid) {
+__device__ __forceinline__ void ns_load(const FsshNArgs* Ap, LaneN<NM, R>& L, int64_t tid, const double* tabs) {
     const FsshNArgs& A = *ns_opaque(Ap);
     constexpr int NP = LaneN<NM, R>::NP;
     const int64_t nt = A.ntraj;
     L.tid = tid;
     const int mid = A.model_id ? A.model_id[tid] : 0;
     L.n = A.slot_n[mid];
-    L.tab = A.slot_tab[mid] >= 0 ? A.mtab + A.slot_tab[mid] : nullptr;
+    L.tab = A.slot_tab[mid] >= 0 ? tabs + A.slot_tab[mid] : nullptr;
     L.m = model_regs(A.models, mid);
     L.r = (R)A.r0[tid];
     L.v = (R)A.v0[tid];
@@ -507,18 +572,40 @@ __device__ __forceinline__ void ns_finish(const FsshNArgs* Ap, const LaneN<NM, R
     A.nhops[L.tid] = L.nh;
 }
 
-template <int NM, typename R>
-__device__ __forceinline__ void ns_step(const FsshNArgs* Ap, const FsshNArgs& A, LaneN<NM, R>& L) {
+// The launch arguments the step reads, in scalar registers for the whole persistent loop (read per step through the
+// argument pointer, each is a vector-memory round trip with a full wait).
+struct NsHot {
+    int32_t method, rescaling, nsub, save_every, cell_mode, term_kind;
+    int64_t nsteps;
+    double dt, inv_mass, term_value;
+    uint64_t key;
+};
+
+__device__ __forceinline__ NsHot ns_hot(const FsshNArgs& A) {
+    NsHot H;
+    H.method = uniform_sgpr(A.method); H.rescaling = uniform_sgpr(A.rescaling); H.nsub = uniform_sgpr(A.nsub);
+    H.save_every = uniform_sgpr(A.save_every); H.cell_mode = uniform_sgpr(A.cell.mode);
+    H.term_kind = uniform_sgpr(A.term_kind); H.nsteps = uniform_sgpr(A.nsteps);
+    H.dt = uniform_sgpr(A.dt); H.inv_mass = uniform_sgpr(A.inv_mass); H.term_value = uniform_sgpr(A.term_value);
+    H.key = uniform_sgpr(A.key);
+    return H;
+}
+
+// SER: the default five sub-steps, by the power series where it serves; otherwise any number of sub-steps.
+template <int NM, typename R, bool SER>
+__device__ __forceinline__ void ns_step(const FsshNArgs* Ap, const FsshNArgs& A, const NsHot& H, LaneN<NM, R>& L) {
     constexpr int NP = LaneN<NM, R>::NP;
     constexpr int NQ = NP > 0 ? NP : 1;
-    const R hdt = (R)(0.5 * A.dt), dtR = (R)A.dt;
+    const R hdt = (R)(0.5 * H.dt), dtR = (R)H.dt;
     const R vt = L.v + hdt * L.k;                                     // step_B!
     L.r = L.r + dtR * vt;                                             // step_A!
     double vd[NM], vo[NQ], dd[NM], dof[NQ], E[NM], Gd[NM], Go[NQ];
     ns_model<NM, R>(L, L.r, vd, vo, dd, dof);                         // update_cache!
+    // from the identity, not from the previous step's basis: where two states cross with a coupling of 1e-20 the sign
+    // of their overlaps hangs on components that small, which rotations of V itself give to full relative accuracy
     ns_eigen<NM>(L.n, vd, vo, E, L.U, true);
     ns_rotate<NM>(L.U, dd, dof, Gd, Go);
-    ns_accel<NM, R>(A, L, Gd, Go, L.a, L.x);                          // sigma of the step start
+    ns_accel<NM, R>(H, L, Gd, Go, L.a, L.x);                          // sigma of the step start
     L.v = vt + hdt * L.k;                                             // step_B!
     // nonadiabatic couplings d_ij = G_ij / (E_j - E_i) and W = v d on the trajectory's n states
     double d[NQ];
@@ -528,21 +615,74 @@ __device__ __forceinline__ void ns_step(const FsshNArgs* Ap, const FsshNArgs& A,
 #pragma unroll
         for (int j = i + 1; j < NM; ++j) {
             const int p = pidx<NM>(i, j);
-            d[p] = (j < L.n) ? Go[p] / (E[j] - E[i]) : 0.0;
+            d[p] = (j < L.n) ? Go[p] * nr_rcp(E[j] - E[i]) : 0.0;
             I.Wn[p] = d[p] * (double)L.v;
             I.Wc[p] = L.Wc[p];
         }
 #pragma unroll
     for (int i = 0; i < NM; ++i) { I.Ec[i] = L.Ec[i]; I.En[i] = E[i]; }
-    const double tn = L.t + A.dt;
+    const double tn = L.t + H.dt;
     I.tc = L.tc; I.tn = tn;
-    {   // step!(electronic_integrator, dt, true): nsub sub-steps clipped to t + dt (bab_electronics.jl:87-90)
-        const double h = A.dt / (double)A.nsub;
-        double tau = L.t;
-        for (int s = 0; s < A.nsub; ++s) {
-            const double hs = fmin(h, tn - tau);
-            ns_tsit5<NM>(I, tau, hs, L.a, L.x, L.y);
-            tau = (s == A.nsub - 1) ? tn : tau + hs;
+    // step!(electronic_integrator, dt, true) (bab_electronics.jl:87-90)
+    bool series = SER;
+    if constexpr (SER) {
+        // energies and couplings at the step start and their change over the step, times dt
+        const double inv = nr_rcp(tn - L.tc), off = (L.t - L.tc) * inv, len = H.dt * inv;
+        double e0[NM], w0[NQ], e1[NM], w1[NQ];
+#pragma unroll
+        for (int i = 0; i < NM; ++i) {
+            const double d1 = E[i] - L.Ec[i];
+            e0[i] = H.dt * fma(d1, off, L.Ec[i]);
+            e1[i] = (H.dt * len) * d1;
+        }
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            const double d1 = I.Wn[p] - L.Wc[p];
+            w0[p] = H.dt * fma(d1, off, L.Wc[p]);
+            w1[p] = (H.dt * len) * d1;
+        }
+        const double m0 = ns_norm<NM>(L.n, e0, w0), m1 = ns_norm<NM>(L.n, e1, w1);
+        const double z2 = fma(4.0, m1, m0 * m0);
+        int parts = 1;
+        if constexpr (sizeof(R) == 8) {
+            // FP64 nuclei: where the sub-steps' own error and theirs on the change of A stay below 1e-12 a step
+            // (series_step2's comment), so that leaving both out changes nothing; else the sub-steps
+            const double m = m0 + m1, mm = m * m;
+            series = 1.4e-8 * (mm * mm) * (mm + m1) < 1e-12;
+        } else {
+            // FP32 nuclei: the series throughout, on parts of the step beyond z2 = 4
+            if (z2 >= 4.0) parts = (int)fmin(ceil(0.5 * sqrt(z2)), 64.0);
+        }
+        if (series) {
+            if constexpr (sizeof(R) == 8) {
+                ns_series<NM>(e0, w0, e1, w1, ns_series_orders(z2), L.a, L.x, L.y);
+            } else {
+                const double rp = nr_rcp((double)parts);
+                const int orders = ns_series_orders(z2 * rp * rp);
+#pragma unroll
+                for (int i = 0; i < NM; ++i) { e0[i] *= rp; e1[i] *= rp * rp; }
+#pragma unroll
+                for (int p = 0; p < NP; ++p) { w0[p] *= rp; w1[p] *= rp * rp; }
+#pragma unroll 1
+                for (int q = 0; q < parts; ++q) {
+                    ns_series<NM>(e0, w0, e1, w1, orders, L.a, L.x, L.y);
+#pragma unroll
+                    for (int i = 0; i < NM; ++i) e0[i] += e1[i];
+#pragma unroll
+                    for (int p = 0; p < NP; ++p) w0[p] += w1[p];
+                }
+            }
+        }
+    }
+    if constexpr (!SER || sizeof(R) == 8) {
+        if (!series) {   // nsub sub-steps clipped to t + dt
+            const double h = H.dt / (double)H.nsub;
+            double tau = L.t;
+            for (int s = 0; s < H.nsub; ++s) {
+                const double hs = fmin(h, tn - tau);
+                ns_tsit5<NM>(I, tau, hs, L.a, L.x, L.y);
+                tau = (s == H.nsub - 1) ? tn : tau + hs;
+            }
         }
     }
 #pragma unroll
@@ -552,8 +692,8 @@ __device__ __forceinline__ void ns_step(const FsshNArgs* Ap, const FsshNArgs& A,
     L.tc = tn;
     L.t = tn;
     // the save precedes the hop callback (a save time holds the state before the step's callbacks)
-    if (A.save_every > 0 && ((L.step + 1) % A.save_every) == 0) ns_save<NM, R>(Ap, L, (L.step + 1) / A.save_every);
-    if (A.method == 0) {  // HoppingCallback (surface_hopping.jl:2-16), fssh.jl:96-121
+    if (H.save_every > 0 && ((L.step + 1) % H.save_every) == 0) ns_save<NM, R>(Ap, L, (L.step + 1) / H.save_every);
+    if (H.method == 0) {  // HoppingCallback (surface_hopping.jl:2-16), fssh.jl:96-121
         const int s = L.st;
         double ass = 0.0;
 #pragma unroll
@@ -572,14 +712,14 @@ __device__ __forceinline__ void ns_step(const FsshNArgs* Ap, const FsshNArgs& A,
                         else if (m > q) { xms = L.x[pidx<NM>(q, m)]; dsm = d[pidx<NM>(q, m)]; }
                     }
                 }
-                pm = 2.0 * (double)L.v * (xms / ass) * dsm * A.dt;
+                pm = 2.0 * (double)L.v * (xms / ass) * dsm * H.dt;
                 pm = fmin(fmax(pm, 0.0), 1.0);
             }
             run += pm;
             cum[m] = run;
         }
         if (run > 0.0) {
-            const double rnd = philox_uniform((uint64_t)L.tid, (uint32_t)L.step, STREAM_HOP, A.key);
+            const double rnd = philox_uniform((uint64_t)L.tid, (uint32_t)L.step, STREAM_HOP, H.key);
             int ns = s;
             bool found = false;
 #pragma unroll
@@ -598,22 +738,25 @@ __device__ __forceinline__ void ns_step(const FsshNArgs* Ap, const FsshNArgs& A,
                 for (int i = 0; i < NM; ++i) { if (i == ns) dE += E[i]; if (i == s) dE -= E[i]; }
                 R vv[1] = {L.v};
                 const double dc[1] = {dno};
-                const double im[1] = {A.inv_mass};
-                if (rescale_velocity<1, R>(A.rescaling, vv, im, dc, dE)) { L.st = ns; ++L.nh; }
+                const double im[1] = {H.inv_mass};
+                if (rescale_velocity<1, R>(H.rescaling, vv, im, dc, dE)) { L.st = ns; ++L.nh; }
                 L.v = vv[0];
             }
         }
     }
-    if (A.cell.mode == 1) {  // CellBoundaryCallback after the hop callback; the step-end acceleration is kept
+    if (H.cell_mode == 1) {  // CellBoundaryCallback after the hop callback; the step-end acceleration is kept
         R rr[1] = {L.r};
         if (cell_outside<1, 1, R>(A.cell, rr)) { cell_wrap<1, 1, R>(A.cell, rr); L.r = rr[0]; }
     }
     ++L.step;
 }
 
-template <int NM, typename R>
-__device__ __forceinline__ void ns_body(const FsshNArgs* __restrict__ Ap) {
+template <int NM, typename R, bool SER>
+__device__ __forceinline__ void ns_body(const FsshNArgs* __restrict__ Ap, double* tabs) {
     const FsshNArgs& A = *Ap;
+    const NsHot H = ns_hot(A);
+    for (int i = threadIdx.x; i < A.ntab; i += blockDim.x) tabs[i] = A.mtab[i];   // the models' tables, read every step
+    __syncthreads();
     const int lane = __lane_id();
     const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     LaneN<NM, R> L;
@@ -630,8 +773,8 @@ __device__ __forceinline__ void ns_body(const FsshNArgs* __restrict__ Ap) {
                 const unsigned long long q = base + (unsigned long long)__popcll(want & below);
                 if (q < (unsigned long long)A.ntraj) {
                     const int32_t* order = ns_opaque(Ap)->order;
-                    ns_load<NM, R>(Ap, L, order ? (int64_t)order[q] : (int64_t)q);
-                    if (A.nsteps <= 0) ns_finish<NM, R>(Ap, L); else active = true;
+                    ns_load<NM, R>(Ap, L, order ? (int64_t)order[q] : (int64_t)q, tabs);
+                    if (H.nsteps <= 0) ns_finish<NM, R>(Ap, L); else active = true;
                 } else {
                     exhausted = true;
                 }
@@ -639,11 +782,11 @@ __device__ __forceinline__ void ns_body(const FsshNArgs* __restrict__ Ap) {
         }
         if (__ballot(active) == 0) break;
         if (active) {
-            ns_step<NM, R>(Ap, A, L);
+            ns_step<NM, R, SER>(Ap, A, H, L);
             // TerminatingCallback after each step, not at t0 (callbacks.jl:15-29)
             const R rr[1] = {L.r};
-            if (L.step >= A.nsteps || (A.cell.mode == 2 && cell_outside<1, 1, R>(A.cell, rr)) ||
-                term_hit(A.term_kind, (double)L.r, A.term_value)) {
+            if (L.step >= H.nsteps || (H.cell_mode == 2 && cell_outside<1, 1, R>(A.cell, rr)) ||
+                term_hit(H.term_kind, (double)L.r, H.term_value)) {
                 ns_finish<NM, R>(Ap, L);
                 active = false;
             }
@@ -651,12 +794,22 @@ __device__ __forceinline__ void ns_body(const FsshNArgs* __restrict__ Ap) {
     }
 }
 
-#define NQCD_NS_KERNELS(NM)                                                                              \
-    __global__ __launch_bounds__(256) void fssh_n_f64_##NM(const FsshNArgs* __restrict__ Ap) {           \
-        ns_body<NM, double>(Ap);                                                                         \
-    }                                                                                                    \
-    __global__ __launch_bounds__(256) void fssh_n_f32_##NM(const FsshNArgs* __restrict__ Ap) {           \
-        ns_body<NM, float>(Ap);                                                                          \
+// f32s, f64s: the default five sub-steps (the power series); f32, f64: other counts.
+#define NQCD_NS_KERNEL(NAME, NM, R, SER)                                                                 \
+    __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((NM) <= 3 ? 2 : 1)))            \
+    void NAME(const FsshNArgs* __restrict__ Ap) {                                                        \
+        extern __shared__ double ns_tabs[];                                                              \
+        ns_body<NM, R, SER>(Ap, ns_tabs);                                                                \
     }
+#define NQCD_NS_KERNELS(NM)                                                                              \
+    NQCD_NS_KERNEL(fssh_n_f64_##NM, NM, double, false)                                                   \
+    NQCD_NS_KERNEL(fssh_n_f64s_##NM, NM, double, true)                                                   \
+    NQCD_NS_KERNEL(fssh_n_f32_##NM, NM, float, false)                                                    \
+    NQCD_NS_KERNEL(fssh_n_f32s_##NM, NM, float, true)
+
+// The kernel of a precision and of the default (five) or another count of sub-steps.
+#define NQCD_NS_PICK(NM, precision, five)                                                                \
+    ((precision) == 0 ? ((five) ? (NsKernelPtr)fssh_n_f64s_##NM : (NsKernelPtr)fssh_n_f64_##NM)                \
+                      : ((five) ? (NsKernelPtr)fssh_n_f32s_##NM : (NsKernelPtr)fssh_n_f32_##NM))
 
 }  // namespace nqcd

@@ -322,6 +322,18 @@ __device__ __forceinline__ ModelLane<R> model_lane(const ModelRegs& m) {
     return L;
 }
 
+// 1/x and 1/sqrt(x) from the hardware estimate and two Newton-Raphson corrections (within an ulp or so).
+__device__ __forceinline__ double nr_rcp(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(r, fma(-x, r, 1.0), r);
+    return fma(r, fma(-x, r, 1.0), r);
+}
+__device__ __forceinline__ double nr_rsq(double x) {
+    double r = __builtin_amdgcn_rsq(x);
+    r = fma(0.5 * r, fma(-x * r, r, 1.0), r);
+    return fma(0.5 * r, fma(-x * r, r, 1.0), r);
+}
+
 // ---------------------------------------------------------------------------
 // 2x2 real symmetric eigen-decomposition, eigenvalues ascending.  U is stored
 // row-major (U[0]=U00, U[1]=U01, U[2]=U10, U[3]=U11); column j is the eigenvector
