@@ -196,7 +196,7 @@ void nqcd_mi355x_close(nqcd_handle_t* h) {
                       &h->r0, &h->v0, &h->sig0, &h->state0, &h->model_id, &h->order, &h->models_dev, &h->bath, &h->inv_mass_dev, &h->args_dev,
                       &h->r, &h->v, &h->sig, &h->state, &h->steps, &h->nhops, &h->save_ad, &h->save_di,
                       &h->save_state, &h->queue, &h->plainS, &h->plainSi, &h->tmp, &h->partial, &h->small, &h->save_centroid, &h->sum64,
-                      &h->save_ekin, &h->save_epot, &h->ns_tab_dev, &h->final_di, &h->save_v, &h->susp_f[0],
+                      &h->save_ekin, &h->save_epot, &h->ns_tab_dev, &h->final_di, &h->save_v, &h->stage, &h->susp_f[0],
                       &h->susp_f[1], &h->susp_tid[0], &h->susp_tid[1], &h->susp_i[0], &h->susp_i[1], &h->susp_ctr};
     for (DevBuf* b : bufs) b->release();
     (void)hipEventDestroy(h->ev0);
@@ -909,34 +909,17 @@ int32_t nqcd_mi355x_download(nqcd_handle_t* h, int32_t field, void* out, int64_t
         field != NQCD_FIELD_SAVE_R && field != NQCD_FIELD_SAVE_V && field != NQCD_FIELD_SAVE_EKIN &&
         field != NQCD_FIELD_SAVE_EPOT)
         return fail(h, NQCD_ERR_UNSUPPORTED, "classical fields: R, V, STEPS, SAVE_R, SAVE_V, SAVE_EKIN, SAVE_EPOT");
-    auto fetch = [&](const DevBuf& b, size_t sz, std::vector<char>& host) -> hipError_t {
-        host.resize(sz);
-        return hipMemcpy(host.data(), b.p, sz, hipMemcpyDeviceToHost);
-    };
-    std::vector<char> raw;
+    double* const o = static_cast<double*>(out);
     switch (field) {
     case NQCD_FIELD_R:
     case NQCD_FIELD_V: {
         if (bytes != (int64_t)sizeof(double) * D * nt) return fail(h, NQCD_ERR_ARG, "bytes mismatch");
-        HIPCHK(h, fetch(field == NQCD_FIELD_R ? h->r : h->v, sizeof(double) * D * nt, raw));
-        const double* s = reinterpret_cast<const double*>(raw.data());
-        double* o = static_cast<double*>(out);
-        for (int64_t i = 0; i < nt; ++i)
-            for (int I = 0; I < D; ++I) o[(size_t)i * D + I] = s[(size_t)I * nt + i];
-        return NQCD_OK;
+        return download_rows(h, field == NQCD_FIELD_R ? h->r : h->v, 0, D, o);
     }
     case NQCD_FIELD_SIGMA_RE:
     case NQCD_FIELD_SIGMA_IM: {
         if (bytes != (int64_t)sizeof(double) * n * n * nt) return fail(h, NQCD_ERR_ARG, "bytes mismatch");
-        HIPCHK(h, fetch(h->sig, sizeof(double) * 4 * nt, raw));
-        const double* s = reinterpret_cast<const double*>(raw.data());
-        double* o = static_cast<double*>(out);
-        for (int64_t i = 0; i < nt; ++i) {
-            double* m = o + (size_t)i * 4;
-            if (field == NQCD_FIELD_SIGMA_RE) { m[0] = s[i]; m[3] = s[nt + i]; m[1] = m[2] = s[2 * nt + i]; }
-            else { m[0] = m[3] = 0.0; m[2] = s[3 * nt + i]; m[1] = -s[3 * nt + i]; }
-        }
-        return NQCD_OK;
+        return download_density2(h, field == NQCD_FIELD_SIGMA_IM, o);
     }
     case NQCD_FIELD_STATE:
     case NQCD_FIELD_STEPS:
@@ -949,45 +932,23 @@ int32_t nqcd_mi355x_download(nqcd_handle_t* h, int32_t field, void* out, int64_t
     case NQCD_FIELD_SAVE_POP_AD:
     case NQCD_FIELD_SAVE_POP_DI: {
         if (bytes != (int64_t)sizeof(double) * n * ns * nt) return fail(h, NQCD_ERR_ARG, "bytes mismatch");
-        HIPCHK(h, fetch(field == NQCD_FIELD_SAVE_POP_AD ? h->save_ad : h->save_di, sizeof(double) * n * ns * nt, raw));
-        const double* s = reinterpret_cast<const double*>(raw.data());
-        double* o = static_cast<double*>(out);
-        for (int64_t i = 0; i < nt; ++i)
-            for (int sl = 0; sl < ns; ++sl)
-                for (int c = 0; c < n; ++c) o[((size_t)i * ns + sl) * n + c] = s[((size_t)sl * n + c) * nt + i];
-        return NQCD_OK;
+        return download_rows(h, field == NQCD_FIELD_SAVE_POP_AD ? h->save_ad : h->save_di, 0, n * ns, o);
     }
     case NQCD_FIELD_SAVE_CENTROID: {
         if (!is_rp(h)) return fail(h, NQCD_ERR_UNSUPPORTED, "centroids exist for ring-polymer problems only");
         if (bytes != (int64_t)sizeof(double) * ns * nt) return fail(h, NQCD_ERR_ARG, "bytes mismatch");
-        HIPCHK(h, fetch(h->save_centroid, sizeof(double) * ns * nt, raw));
-        const double* s = reinterpret_cast<const double*>(raw.data());
-        double* o = static_cast<double*>(out);
-        for (int64_t i = 0; i < nt; ++i)
-            for (int sl = 0; sl < ns; ++sl) o[(size_t)i * ns + sl] = s[(size_t)sl * nt + i];
-        return NQCD_OK;
+        return download_rows(h, h->save_centroid, 0, ns, o);
     }
     case NQCD_FIELD_SAVE_V: {
         if (!cls_is_problem(h)) return fail(h, NQCD_ERR_UNSUPPORTED, "velocities per save exist for classical problems");
         if (bytes != (int64_t)sizeof(double) * ns * nt) return fail(h, NQCD_ERR_ARG, "bytes mismatch");
-        HIPCHK(h, fetch(h->save_v, sizeof(double) * ns * nt, raw));
-        const double* s = reinterpret_cast<const double*>(raw.data());
-        double* o = static_cast<double*>(out);
-        for (int64_t i = 0; i < nt; ++i)
-            for (int sl = 0; sl < ns; ++sl) o[(size_t)i * ns + sl] = s[(size_t)sl * nt + i];
-        return NQCD_OK;
+        return download_rows(h, h->save_v, 0, ns, o);
     }
     case NQCD_FIELD_SAVE_R: {
         if (!nd_is_problem(h) && !cme_is_problem(h) && !cls_is_problem(h))
             return fail(h, NQCD_ERR_UNSUPPORTED, "configurations per save exist for the diatom-surface and CME models");
         if (bytes != (int64_t)sizeof(double) * D * ns * nt) return fail(h, NQCD_ERR_ARG, "bytes mismatch");
-        HIPCHK(h, fetch(h->save_centroid, sizeof(double) * D * ns * nt, raw));
-        const double* s = reinterpret_cast<const double*>(raw.data());
-        double* o = static_cast<double*>(out);
-        for (int64_t i = 0; i < nt; ++i)
-            for (int sl = 0; sl < ns; ++sl)
-                for (int I = 0; I < D; ++I) o[((size_t)i * ns + sl) * D + I] = s[((size_t)sl * D + I) * nt + i];
-        return NQCD_OK;
+        return download_rows(h, h->save_centroid, 0, D * ns, o);
     }
     case NQCD_FIELD_FALLBACKS: {
         if (!nd_is_problem(h) || h->models[0].kind != NQCD_MODEL_MLP_SURROGATE)
@@ -1002,31 +963,17 @@ int32_t nqcd_mi355x_download(nqcd_handle_t* h, int32_t field, void* out, int64_t
             (is_rp(h) || nd_is_problem(h) || is_spin_boson(h) || !is_two_state_1d(h)))
             return fail(h, NQCD_ERR_UNSUPPORTED, "energies per save exist for two-state one-dof FSSH / Ehrenfest");
         if (bytes != (int64_t)sizeof(double) * ns * nt) return fail(h, NQCD_ERR_ARG, "bytes mismatch");
-        HIPCHK(h, fetch(field == NQCD_FIELD_SAVE_EKIN ? h->save_ekin : h->save_epot, sizeof(double) * ns * nt, raw));
-        const double* s = reinterpret_cast<const double*>(raw.data());
-        double* o = static_cast<double*>(out);
-        for (int64_t i = 0; i < nt; ++i)
-            for (int sl = 0; sl < ns; ++sl) o[(size_t)i * ns + sl] = s[(size_t)sl * nt + i];
-        return NQCD_OK;
+        return download_rows(h, field == NQCD_FIELD_SAVE_EKIN ? h->save_ekin : h->save_epot, 0, ns, o);
     }
     case NQCD_FIELD_FINAL_POP_DI: {
         if (!is_two_state_1d(h))
             return fail(h, NQCD_ERR_UNSUPPORTED, "diabatic final populations exist for two-state one-dof FSSH / Ehrenfest");
         if (bytes != (int64_t)sizeof(double) * 2 * nt) return fail(h, NQCD_ERR_ARG, "bytes mismatch");
-        HIPCHK(h, fetch(h->final_di, sizeof(double) * 2 * nt, raw));
-        const double* s = reinterpret_cast<const double*>(raw.data());
-        double* o = static_cast<double*>(out);
-        for (int64_t i = 0; i < nt; ++i) { o[2 * i] = s[i]; o[2 * i + 1] = s[nt + i]; }
-        return NQCD_OK;
+        return download_rows(h, h->final_di, 0, 2, o);
     }
     case NQCD_FIELD_SAVE_STATE: {
         if (bytes != (int64_t)sizeof(int32_t) * ns * nt) return fail(h, NQCD_ERR_ARG, "bytes mismatch");
-        HIPCHK(h, fetch(h->save_state, sizeof(int32_t) * ns * nt, raw));
-        const int32_t* s = reinterpret_cast<const int32_t*>(raw.data());
-        int32_t* o = static_cast<int32_t*>(out);
-        for (int64_t i = 0; i < nt; ++i)
-            for (int sl = 0; sl < ns; ++sl) o[(size_t)i * ns + sl] = s[(size_t)sl * nt + i];
-        return NQCD_OK;
+        return download_rows(h, h->save_state, 0, ns, static_cast<int32_t*>(out));
     }
     default: return fail(h, NQCD_ERR_ARG, "unknown field");
     }

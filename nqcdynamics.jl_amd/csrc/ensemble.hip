@@ -11,6 +11,7 @@
 #include <mutex>
 
 #include "ensemble.h"
+#include "handle.h"
 
 namespace nqcd {
 
@@ -293,6 +294,109 @@ hipError_t launch_zero(void* p, size_t bytes, hipStream_t s) {
     const size_t blocks = std::min<size_t>((n + 255) / 256, 8192);
     hipLaunchKernelGGL(zero_words, dim3((unsigned)blocks), dim3(256), 0, s, reinterpret_cast<uint32_t*>(p), n);
     return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// Per-trajectory fields to the host.  The device keeps rows [row][trajectory]; callers get [trajectory][row].  The
+// transposition runs on the device, in 64 x 16 tiles through LDS so that reads along trajectories and writes along
+// rows both move whole segments, into a bounded staging buffer that is copied straight into the caller's array:
+// bound by the copy to the host.  1e5 ring polymers of 32 beads, 1000 steps and their final positions: 10.1 ms with a
+// copy into a host vector and a strided host pass, 4.5 ms here (2.5 of them the steps).
+// ---------------------------------------------------------------------------
+constexpr int kTileT = 64, kTileR = 16;
+// Output row k is source row (k / g) * G + k % g.
+template <typename T>
+__global__ __launch_bounds__(256) void transpose_rows(const T* __restrict__ src, int64_t nt, int32_t g, int32_t G,
+                                                      int32_t rows, int64_t t0, int64_t cnt, T* __restrict__ out) {
+    __shared__ T tile[kTileR][kTileT + 1];
+    const int64_t tb = (int64_t)blockIdx.x * kTileT;
+    const int tl = threadIdx.x & 63, rl = threadIdx.x >> 6;
+    const int rw = threadIdx.x & 15, tw = threadIdx.x >> 4;
+    for (int32_t rb = 0; rb < rows; rb += kTileR) {
+#pragma unroll
+        for (int k = 0; k < kTileR; k += 4) {
+            const int32_t r = rb + rl + k;
+            if (r < rows && tb + tl < cnt) tile[rl + k][tl] = src[((int64_t)(r / g) * G + r % g) * nt + t0 + tb + tl];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kTileT; k += 16)
+            if (rb + rw < rows && tb + tw + k < cnt) out[(tb + tw + k) * (int64_t)rows + rb + rw] = tile[rw][tw + k];
+        __syncthreads();
+    }
+}
+
+// The real or imaginary part of the 2 x 2 density matrices (column-major) from the rows s00, s11, Re s01, Im s01.
+__global__ __launch_bounds__(256) void expand_density2(const double* __restrict__ sig, int64_t nt, int32_t im, int64_t t0,
+                                                       int64_t cnt, double* __restrict__ out) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= cnt) return;
+    double* m = out + 4 * i;
+    if (im) {
+        const double y = sig[3 * nt + t0 + i];
+        m[0] = 0.0; m[1] = -y; m[2] = y; m[3] = 0.0;
+    } else {
+        const double x = sig[2 * nt + t0 + i];
+        m[0] = sig[t0 + i]; m[1] = x; m[2] = x; m[3] = sig[nt + t0 + i];
+    }
+}
+
+// Runs fill(t0, cnt, staging) over chunks of trajectories, `row_bytes` of output each, and copies every chunk out.
+template <class F>
+static int32_t download_chunks(nqcd_handle_t* h, size_t row_bytes, void* out, F&& fill) {
+    std::lock_guard<std::mutex> lock(h->stage_mu);
+    const int64_t nt = h->ntraj;
+    size_t chunk = std::min<size_t>(std::max<size_t>(kStageBytes / row_bytes, 1), (size_t)nt);
+    if (h->stage.bytes < chunk * row_bytes && h->stage.ensure(chunk * row_bytes) != hipSuccess) {
+        (void)hipGetLastError();   // a nearly full device: one megabyte (or a single trajectory) at a time
+        chunk = std::min<size_t>(std::max<size_t>((size_t(1) << 20) / row_bytes, 1), (size_t)nt);
+        HIPCHK(h, h->stage.ensure(chunk * row_bytes));
+    }
+    for (int64_t t0 = 0; t0 < nt; t0 += (int64_t)chunk) {
+        const int64_t cnt = std::min<int64_t>((int64_t)chunk, nt - t0);
+        fill(t0, cnt, h->stage.p);
+        HIPCHK(h, hipGetLastError());
+        HIPCHK(h, hipMemcpyAsync(static_cast<char*>(out) + (size_t)t0 * row_bytes, h->stage.p, (size_t)cnt * row_bytes,
+                                 hipMemcpyDeviceToHost, h->stream));
+        HIPCHK(h, hipStreamSynchronize(h->stream));
+    }
+    return NQCD_OK;
+}
+
+template <typename T>
+static int32_t download_rows_t(nqcd_handle_t* h, const DevBuf& b, int32_t first, int32_t g, int32_t G, int32_t rows, T* out) {
+    if (rows <= 0 || h->ntraj <= 0) return NQCD_OK;
+    const size_t end = (size_t)first + (size_t)((rows - 1) / g) * G + (rows - 1) % g + 1;
+    if (!b.p || b.bytes < sizeof(T) * end * (size_t)h->ntraj) return fail(h, NQCD_ERR_STATE, "this run kept no such field");
+    const T* src = b.as<T>() + (size_t)first * h->ntraj;
+    if (rows == 1) {
+        HIPCHK(h, hipMemcpyAsync(out, src, sizeof(T) * (size_t)h->ntraj, hipMemcpyDeviceToHost, h->stream));
+        HIPCHK(h, hipStreamSynchronize(h->stream));
+        return NQCD_OK;
+    }
+    return download_chunks(h, sizeof(T) * (size_t)rows, out, [&](int64_t t0, int64_t cnt, void* stage) {
+        hipLaunchKernelGGL(transpose_rows<T>, dim3((unsigned)((cnt + kTileT - 1) / kTileT)), dim3(256), 0, h->stream, src,
+                           h->ntraj, g, G, rows, t0, cnt, static_cast<T*>(stage));
+    });
+}
+
+int32_t download_rows(nqcd_handle_t* h, const DevBuf& src, int32_t first, int32_t rows, double* out) {
+    return download_rows_t<double>(h, src, first, rows, rows, rows, out);
+}
+int32_t download_rows(nqcd_handle_t* h, const DevBuf& src, int32_t first, int32_t rows, int32_t* out) {
+    return download_rows_t<int32_t>(h, src, first, rows, rows, rows, out);
+}
+int32_t download_row_groups(nqcd_handle_t* h, const DevBuf& src, int32_t first, int32_t g, int32_t G, int32_t rows, double* out) {
+    return download_rows_t<double>(h, src, first, g, G, rows, out);
+}
+int32_t download_density2(nqcd_handle_t* h, bool im, double* out) {
+    if (h->ntraj <= 0) return NQCD_OK;
+    if (!h->sig.p || h->sig.bytes < sizeof(double) * 4 * (size_t)h->ntraj)
+        return fail(h, NQCD_ERR_STATE, "this run kept no density matrices");
+    return download_chunks(h, 4 * sizeof(double), out, [&](int64_t t0, int64_t cnt, void* stage) {
+        hipLaunchKernelGGL(expand_density2, dim3(grid_for(cnt, 256)), dim3(256), 0, h->stream, h->sig.as<double>(), h->ntraj,
+                           im ? 1 : 0, t0, cnt, static_cast<double*>(stage));
+    });
 }
 
 }  // namespace nqcd

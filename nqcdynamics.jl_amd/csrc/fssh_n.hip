@@ -278,11 +278,6 @@ int32_t ns_download(nqcd_handle_t* h, int32_t field, void* out, int64_t bytes) {
     auto need = [&](int64_t b) -> int32_t {
         return b == bytes ? NQCD_OK : fail(h, NQCD_ERR_ARG, "bytes does not match the field size (" + std::to_string(b) + ")");
     };
-    std::vector<double> tmp;
-    auto fetch = [&](const void* src, size_t count) -> hipError_t {
-        tmp.resize(count);
-        return hipMemcpy(tmp.data(), src, sizeof(double) * count, hipMemcpyDeviceToHost);
-    };
     switch (field) {
     case NQCD_FIELD_R:
     case NQCD_FIELD_V: {
@@ -293,13 +288,8 @@ int32_t ns_download(nqcd_handle_t* h, int32_t field, void* out, int64_t bytes) {
     case NQCD_FIELD_SIGMA_RE:
     case NQCD_FIELD_SIGMA_IM: {
         if (int32_t rc = need(8 * (int64_t)n * n * nt)) return rc;
-        const double* src = h->sig.as<double>() + (field == NQCD_FIELD_SIGMA_IM ? (size_t)NM * NM * nt : 0);
-        HIPCHK(h, fetch(src, (size_t)NM * NM * nt));
-        double* o = static_cast<double*>(out);
-        for (int64_t t = 0; t < nt; ++t)
-            for (int j = 0; j < n; ++j)
-                for (int i = 0; i < n; ++i) o[(size_t)t * n * n + i + (size_t)n * j] = tmp[(size_t)(i + NM * j) * nt + t];
-        return NQCD_OK;
+        return download_row_groups(h, h->sig, field == NQCD_FIELD_SIGMA_IM ? NM * NM : 0, n, NM, n * n,
+                                   static_cast<double*>(out));
     }
     case NQCD_FIELD_STATE:
     case NQCD_FIELD_STEPS:
@@ -312,21 +302,12 @@ int32_t ns_download(nqcd_handle_t* h, int32_t field, void* out, int64_t bytes) {
     case NQCD_FIELD_SAVE_POP_AD:
     case NQCD_FIELD_SAVE_POP_DI: {
         if (int32_t rc = need(8 * (int64_t)n * ns * nt)) return rc;
-        HIPCHK(h, fetch(field == NQCD_FIELD_SAVE_POP_AD ? h->save_ad.p : h->save_di.p, (size_t)NM * ns * nt));
-        double* o = static_cast<double*>(out);
-        for (int64_t t = 0; t < nt; ++t)
-            for (int s = 0; s < ns; ++s)
-                for (int i = 0; i < n; ++i) o[((size_t)t * ns + s) * n + i] = tmp[((size_t)s * NM + i) * nt + t];
-        return NQCD_OK;
+        return download_row_groups(h, field == NQCD_FIELD_SAVE_POP_AD ? h->save_ad : h->save_di, 0, n, NM, n * ns,
+                                   static_cast<double*>(out));
     }
     case NQCD_FIELD_SAVE_STATE: {
         if (int32_t rc = need(4 * (int64_t)ns * nt)) return rc;
-        std::vector<int32_t> ti((size_t)ns * nt);
-        HIPCHK(h, hipMemcpy(ti.data(), h->save_state.p, 4 * (size_t)ns * nt, hipMemcpyDeviceToHost));
-        int32_t* o = static_cast<int32_t*>(out);
-        for (int64_t t = 0; t < nt; ++t)
-            for (int s = 0; s < ns; ++s) o[(size_t)t * ns + s] = ti[(size_t)s * nt + t];
-        return NQCD_OK;
+        return download_rows(h, h->save_state, 0, ns, static_cast<int32_t*>(out));
     }
     default: return fail(h, NQCD_ERR_UNSUPPORTED, "field not available for n-state problems");
     }

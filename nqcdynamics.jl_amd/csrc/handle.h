@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -29,6 +30,14 @@ struct DevBuf {
 };
 
 int32_t fail(nqcd_handle_t* h, int32_t code, const std::string& msg);
+
+// Per-trajectory fields to the host: `rows` device rows [row][trajectory] from row `first` on as [trajectory][row] (ensemble.hip); of a
+// group of G device rows, the first g (n-state kernels of more states than the problem); the two-state densities.
+constexpr size_t kStageBytes = size_t(64) << 20;   // most of the staging buffer a handle keeps for these
+int32_t download_rows(nqcd_handle_t* h, const DevBuf& src, int32_t first, int32_t rows, double* out);
+int32_t download_rows(nqcd_handle_t* h, const DevBuf& src, int32_t first, int32_t rows, int32_t* out);
+int32_t download_row_groups(nqcd_handle_t* h, const DevBuf& src, int32_t first, int32_t g, int32_t G, int32_t rows, double* out);
+int32_t download_density2(nqcd_handle_t* h, bool im, double* out);
 
 }  // namespace nqcd
 
@@ -83,6 +92,8 @@ struct nqcd_handle {
     nqcd::DevBuf r0, v0, sig0, state0, model_id, order, models_dev, bath, inv_mass_dev, args_dev;
     nqcd::DevBuf r, v, sig, state, steps, nhops, save_ad, save_di, save_state;
     nqcd::DevBuf queue, plainS, plainSi, tmp, partial, small, save_centroid, sum64, save_ekin, save_epot, final_di;
+    nqcd::DevBuf stage;    // transposed fields on their way to the host
+    std::mutex stage_mu;   // several threads may read one handle's results
     nqcd::DevBuf save_v;   // velocities per save (classical dynamics)
     // trajectories set aside between the launches of a persistent two-state run (two sets used in turn)
     nqcd::DevBuf susp_f[2], susp_tid[2], susp_i[2], susp_ctr;

@@ -1497,14 +1497,8 @@ int32_t ie_download(nqcd_handle_t* h, int32_t field, void* out, int64_t bytes) {
     case NQCD_FIELD_SAVE_POP_AD:
     case NQCD_FIELD_SAVE_POP_DI: {  // (N, nsave, ntraj)
         if (bytes != (int64_t)sizeof(double) * N * ns * nt) return fail(h, NQCD_ERR_ARG, "bytes mismatch");
-        std::vector<double> t((size_t)N * ns * nt);
-        HIPCHK(h, hipMemcpy(t.data(), field == NQCD_FIELD_SAVE_POP_AD ? h->save_ad.p : h->save_di.p,
-                            sizeof(double) * t.size(), hipMemcpyDeviceToHost));
-        double* o = static_cast<double*>(out);
-        for (int64_t i = 0; i < nt; ++i)
-            for (int sl = 0; sl < ns; ++sl)
-                for (int a = 0; a < N; ++a) o[((size_t)i * ns + sl) * N + a] = t[((size_t)sl * N + a) * nt + i];
-        return NQCD_OK;
+        return download_rows(h, field == NQCD_FIELD_SAVE_POP_AD ? h->save_ad : h->save_di, 0, N * ns,
+                             static_cast<double*>(out));
     }
     default: return fail(h, NQCD_ERR_UNSUPPORTED, "field not available for IESH / EhrenfestNA");
     }

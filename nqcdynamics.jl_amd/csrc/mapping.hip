@@ -766,28 +766,17 @@ int32_t map_download(nqcd_handle_t* h, int32_t field, void* out, int64_t bytes) 
     auto need = [&](int64_t b) -> int32_t {
         return b == bytes ? NQCD_OK : fail(h, NQCD_ERR_ARG, "bytes does not match the field size (" + std::to_string(b) + ")");
     };
-    std::vector<double> tmp;
-    auto fetch = [&](const void* src, size_t count) -> hipError_t {
-        tmp.resize(count);
-        return hipMemcpy(tmp.data(), src, sizeof(double) * count, hipMemcpyDeviceToHost);
-    };
     double* o = static_cast<double*>(out);
     switch (field) {
     case NQCD_FIELD_R:
     case NQCD_FIELD_V: {   // (nbeads, ntraj)
         if (int32_t rc = need(8 * (int64_t)B * nt)) return rc;
-        HIPCHK(h, fetch(field == NQCD_FIELD_R ? h->r.p : h->v.p, (size_t)B * nt));
-        for (int64_t t = 0; t < nt; ++t)
-            for (int b = 0; b < B; ++b) o[(size_t)t * B + b] = tmp[(size_t)b * nt + t];
-        return NQCD_OK;
+        return download_rows(h, field == NQCD_FIELD_R ? h->r : h->v, 0, B, o);
     }
     case NQCD_FIELD_SAVE_CENTROID: {
         if (!map_rp(h)) return fail(h, NQCD_ERR_UNSUPPORTED, "centroids exist for ring polymers");
         if (int32_t rc = need(8 * (int64_t)ns * nt)) return rc;
-        HIPCHK(h, fetch(h->save_centroid.p, (size_t)ns * nt));
-        for (int64_t t = 0; t < nt; ++t)
-            for (int s = 0; s < ns; ++s) o[(size_t)t * ns + s] = tmp[(size_t)s * nt + t];
-        return NQCD_OK;
+        return download_rows(h, h->save_centroid, 0, ns, o);
     }
     case NQCD_FIELD_STEPS: {
         if (int32_t rc = need(4 * nt)) return rc;
@@ -798,33 +787,20 @@ int32_t map_download(nqcd_handle_t* h, int32_t field, void* out, int64_t bytes) 
     case NQCD_FIELD_MAP_P: {   // (n, nbeads, ntraj)
         const int rows = n * B;
         if (int32_t rc = need(8 * (int64_t)rows * nt)) return rc;
-        HIPCHK(h, fetch(h->sig.as<double>() + (field == NQCD_FIELD_MAP_P ? (size_t)rows * nt : 0), (size_t)rows * nt));
-        for (int64_t t = 0; t < nt; ++t)
-            for (int i = 0; i < rows; ++i) o[(size_t)t * rows + i] = tmp[(size_t)i * nt + t];
-        return NQCD_OK;
+        return download_rows(h, h->sig, field == NQCD_FIELD_MAP_P ? rows : 0, rows, o);
     }
     case NQCD_FIELD_INIT_POP_DI: {
         if (int32_t rc = need(8 * (int64_t)n * nt)) return rc;
-        HIPCHK(h, fetch(h->final_di.p, (size_t)n * nt));
-        for (int64_t t = 0; t < nt; ++t)
-            for (int i = 0; i < n; ++i) o[(size_t)t * n + i] = tmp[(size_t)i * nt + t];
-        return NQCD_OK;
+        return download_rows(h, h->final_di, 0, n, o);
     }
     case NQCD_FIELD_SAVE_POP_DI: {
         if (int32_t rc = need(8 * (int64_t)n * ns * nt)) return rc;
-        HIPCHK(h, fetch(h->save_di.p, (size_t)n * ns * nt));
-        for (int64_t t = 0; t < nt; ++t)
-            for (int s = 0; s < ns; ++s)
-                for (int i = 0; i < n; ++i) o[((size_t)t * ns + s) * n + i] = tmp[((size_t)s * n + i) * nt + t];
-        return NQCD_OK;
+        return download_rows(h, h->save_di, 0, n * ns, o);
     }
     case NQCD_FIELD_SAVE_EKIN:
     case NQCD_FIELD_SAVE_EPOT: {
         if (int32_t rc = need(8 * (int64_t)ns * nt)) return rc;
-        HIPCHK(h, fetch(field == NQCD_FIELD_SAVE_EKIN ? h->save_ekin.p : h->save_epot.p, (size_t)ns * nt));
-        for (int64_t t = 0; t < nt; ++t)
-            for (int s = 0; s < ns; ++s) o[(size_t)t * ns + s] = tmp[(size_t)s * nt + t];
-        return NQCD_OK;
+        return download_rows(h, field == NQCD_FIELD_SAVE_EKIN ? h->save_ekin : h->save_epot, 0, ns, o);
     }
     default:
         return fail(h, NQCD_ERR_UNSUPPORTED, "mapping fields: R, V, STEPS, MAP_X, MAP_P, INIT_POP_DI, SAVE_POP_DI, SAVE_EKIN, SAVE_EPOT (and SAVE_CENTROID for "
