@@ -183,9 +183,8 @@ __device__ __forceinline__ void surrogate_eval(const FsshNdArgs& A, const unsign
 #pragma unroll
         for (int i = 0; i < kMlpIn; ++i) xs[i] = __shfl(xn[i], sl);
         float o[kMlpOut], Jt[kMlpOut][kMlpIn];
-        mlp_tile<true>(lds + m * kPkBytes, xs, o, Jt);
-        // outputs sit in lanes 0..15 and the gradient in every lane of the sample: the owner of
-        // slot 16 T + mj takes those of sample mj
+        mlp_tile<true>(lds + m * kPkBytes, xs, o, Jt, mj);
+        // the owner of slot 16 T + mj takes sample mj (the outputs sit in lanes 0..15)
         const bool mine = active && (mt == T);
 #pragma unroll
         for (int r3 = 0; r3 < kMlpOut; ++r3) {
@@ -194,8 +193,7 @@ __device__ __forceinline__ void surrogate_eval(const FsshNdArgs& A, const unsign
             if (mine && m == 1) H1[r3] = ov;
 #pragma unroll
             for (int i = 0; i < kMlpIn; ++i) {
-                const float gv = __shfl(Jt[r3][i], mj);
-                if (mine) Js[r3][i] += gv;
+                if (mine) Js[r3][i] += Jt[r3][i];
             }
         }
     }

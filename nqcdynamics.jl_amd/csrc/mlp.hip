@@ -151,7 +151,7 @@ __global__ __launch_bounds__(128) void mlp_train_grad(const unsigned char* __res
 #pragma unroll
         for (int i = 0; i < kMlpIn; ++i) xs[i] = valid ? Xn[(int64_t)s * kMlpIn + i] : 0.0f;
         float o[kMlpOut], J[kMlpOut][kMlpIn], h1[32], s1[32], h2[32], s2[32];
-        mlp_tile<false>(S.member, xs, o, J, h1, s1, h2, s2);
+        mlp_tile<false>(S.member, xs, o, J, j, h1, s1, h2, s2);
         // output residuals (sample j lives in lane j of group 0)
         float d3[kMlpOut];
         float lo = 0.0f;
