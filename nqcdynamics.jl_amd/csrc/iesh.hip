@@ -65,25 +65,6 @@ struct IeshArgs {
     double* save_ad;              // (nsave, N, ntraj)
 };
 
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
-}
-
-// Sum over the workgroup, same value returned to every thread; fixed reduction order.
-template <int NT>
-__device__ __forceinline__ double block_sum(double v, double* red) {
-    v = wave_sum(v);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    double s = 0.0;
-#pragma unroll
-    for (int j = 0; j < NT; ++j) s += red[j];
-    return s;
-}
-
 template <int NT>
 __device__ __forceinline__ double block_max(double v, double* red) {
 #pragma unroll
@@ -177,9 +158,9 @@ __device__ double secular_root(const double* eps, int M, int i, double V2, doubl
         if (fabs(f) <= 8.0 * __DBL_EPSILON__ * (fabs(lam) + fabs(h) + V2 * (sl - sh))) break;
         if (f > 0.0) hi = lam;
         else lo = lam;
-        const double bl = has_lo ? -(V2 * sl2 + wl) * (lam - dl) * (lam - dl) : 0.0;
-        const double bh = has_hi ? -(V2 * sh2 + (1.0 - wl)) * (lam - dh) * (lam - dh) : 0.0;
-        const double c = f - (has_lo ? bl / (lam - dl) : 0.0) - (has_hi ? bh / (lam - dh) : 0.0);
+        const double ql = has_lo ? -(V2 * sl2 + wl) * (lam - dl) : 0.0, qh = has_hi ? -(V2 * sh2 + (1.0 - wl)) * (lam - dh) : 0.0;
+        const double bl = ql * (lam - dl), bh = qh * (lam - dh);
+        const double c = f - ql - qh;
         double nl;
         if (has_lo && has_hi) {
             // c t (t - D) + bl (t - D) + bh t = 0 with t = y - dl, D = dh - dl; root in (0, D)
@@ -187,18 +168,34 @@ __device__ double secular_root(const double* eps, int M, int i, double V2, doubl
             const double a1 = bl + bh - c * D, a0 = -bl * D;
             const double sq = sqrt(fmax(a1 * a1 - 4.0 * c * a0, 0.0));
             const double den = a1 > 0.0 ? -a1 - sq : -a1 + sq;
-            nl = dl + den / (2.0 * c);
-            if (!(nl >= lo && nl <= hi)) nl = dl + 2.0 * a0 / den;
+            nl = dl + den * rcp_nr(2.0 * c);
+            if (!(nl >= lo && nl <= hi)) nl = dl + 2.0 * a0 * rcp_nr(den);
         } else if (has_hi) {
-            nl = dh - bh / c;
+            nl = dh - bh * rcp_nr(c);
         } else {
-            nl = dl - bl / c;
+            nl = dl - bl * rcp_nr(c);
         }
         if (fabs(nl - lam) <= 4.0 * __DBL_EPSILON__ * fabs(lam) || (hi - lo) <= tol) break;
         if (!(nl > lo && nl < hi)) nl = 0.5 * (lo + hi);
         lam = nl;
     }
     return lam;
+}
+
+__device__ __forceinline__ double readlane_f64(double x, int lane) {
+    const long long bits = __double_as_longlong(x);
+    const int lo = __builtin_amdgcn_readlane((int)(bits & 0xffffffffll), lane);
+    const int hi = __builtin_amdgcn_readlane((int)(bits >> 32), lane);
+    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
+}
+
+// Sum over the wavefront, the same value in every lane: butterflies inside each row of 16 lanes, then the four rows.
+__device__ __forceinline__ double wave_sum(double v) {
+    v += dpp_f64<0xB1>(v);
+    v += dpp_f64<0x4E>(v);
+    v += dpp_f64<0x141>(v);  // row_half_mirror
+    v += dpp_f64<0x140>(v);  // row_mirror
+    return (readlane_f64(v, 0) + readlane_f64(v, 16)) + (readlane_f64(v, 32) + readlane_f64(v, 48));
 }
 
 // Orders this wavefront's LDS accesses: its lanes exchange data through LDS without a workgroup
@@ -212,14 +209,16 @@ __device__ __forceinline__ void wave_lds_sync() {
 // wins, the lower idx on ties).
 // Eigenvalue ir of the Newns-Anderson matrix at impurity energy h: the secular root on its
 // bracket (the outer brackets reach past the band and h by the coupling norm zn = sqrt(M) V);
-// warm starts from `guess`, a cold start from below the bracket.  Also returns f'(E_ir).
+// warm starts from `guess` (from `prev` where that leaves the bracket), a cold start from below the bracket.
+// Also returns f'(E_ir).
 template <int G = 1>
 __device__ __forceinline__ double na_root(const double* eps, int M, double a, double V2, double zn, double h, int ir,
-                                          bool warm, double guess, double& fp, int sub = 0) {
+                                          bool warm, double guess, double prev, double& fp, int sub = 0) {
     const double lo = (ir == 0) ? fmin(h, eps[0]) - zn - 1e-3 * (zn + 1e-300) : eps[ir - 1];
     const double hi = (ir == M) ? fmax(h, eps[M - 1]) + zn + 1e-3 * (zn + 1e-300) : eps[ir];
     const double scale = fmax(fmax(fabs(a), fabs(eps[M - 1])), fabs(h)) + zn;
-    return secular_root<G>(eps, M, ir, V2, h, lo, hi, warm ? guess : lo - 1.0, 4.0e-16 * scale, fp, sub);
+    return secular_root<G>(eps, M, ir, V2, h, lo, hi, warm ? ((guess > lo && guess < hi) ? guess : prev) : lo - 1.0,
+                           4.0e-16 * scale, fp, sub);
 }
 
 template <int CTRL>
@@ -230,13 +229,6 @@ __device__ __forceinline__ void argmax_dpp(double& mag, int& idx) {
     const int oi = __builtin_amdgcn_update_dpp(0, idx, CTRL, 0xF, 0xF, false);
     const double om = __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
     if (om > mag || (om == mag && oi < idx)) { mag = om; idx = oi; }
-}
-
-__device__ __forceinline__ double readlane_f64(double x, int lane) {
-    const long long bits = __double_as_longlong(x);
-    const int lo = __builtin_amdgcn_readlane((int)(bits & 0xffffffffll), lane);
-    const int hi = __builtin_amdgcn_readlane((int)(bits >> 32), lane);
-    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
 
 // Wavefront-uniform arg-max of (mag, idx), the lowest idx among equal maxima: butterflies inside
@@ -323,9 +315,31 @@ __device__ bool wave_det(double* Sre, double* Sim, int LD, int Ne, double& dre, 
     return true;
 }
 
+// Norms of dt H above which the Taylor series takes another term: the remainder x^(K+1) / (K+1)! e^x of K terms passes
+// 1e-17 at kTaylorFrom[K] (rounded down).  The last entry lies above the 0.5 of a sub-step.
+__constant__ float kTaylorFrom[16] = {
+    9.999990e-18f, 4.472131e-09f, 3.914859e-06f, 1.244626e-04f, 1.036921e-03f, 4.391071e-03f, 1.257669e-02f, 2.812954e-02f,
+    5.324670e-02f, 8.955433e-02f, 1.380727e-01f, 1.992883e-01f, 2.732652e-01f, 3.597589e-01f, 4.583142e-01f, 5.683443e-01f};
+
+// The thread index made opaque where a phase of the step begins: what a phase derives from it (LDS addresses, row
+// and column numbers) is then computed there, instead of being hoisted out of the step loop and held in registers
+// through every other phase.
+__device__ __forceinline__ int ie_tid() {
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
+}
+#define IE_IDS const int tid = ie_tid(), w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63; (void)w; (void)l;
+
+// Bound by the matrix cores in the propagator (8 or 9 terms of N x N x 2 Ne) and, up to 64 states, by the latency of
+// the phases around it, which one workgroup cannot hide: there the registers are held to three wavefronts a SIMD, so
+// that three or four trajectories share a compute unit (those phases were 41 of a step's 57 us at 41 states).  Larger problems fill the LDS with one trajectory and keep two wavefronts' registers.  The phases
+// exchange sums once (coupling norm, hop bound, orbital weight ride on the propagator's registers and barriers) and
+// divide by Newton-Raphson reciprocals.  8192 trajectories of 41 states, 100 steps: 92.3 -> 65.9 ms; 2048 of 101
+// states, 50 steps: 102.5 -> 95.5 ms.
 // RPB: ring polymer (BCBWavefunction), a separate instantiation so the one-bead kernels carry none of it
 template <int NT, int CTM, bool RPB>
-__global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(2))) void iesh_kernel(const IeshArgs A) {
+__global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(NT <= 4 && CTM <= 4 && !RPB ? 3 : 2))) void iesh_kernel(const IeshArgs A) {
     constexpr int NP = 16 * NT;  // padded state count (rows of psi / W tiles)
     constexpr int B = 64 * NT;
     constexpr int KF = 4 * NT;   // A-fragments per lane (K = NP in steps of 4)
@@ -363,6 +377,7 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(2))) vo
     for (int k = tid; k < NP; k += B) eps[k] = (k < M) ? A.a + k * A.de : 0.0;
     __syncthreads();
     const double zn = sqrt((double)M) * A.V;
+    const float order_from = (threadIdx.x & 63) < 16 ? kTaylorFrom[threadIdx.x & 15] : __builtin_inff();
 
     for (int64_t traj = blockIdx.x; traj < A.ntraj; traj += gridDim.x) {
         __syncthreads();
@@ -418,38 +433,44 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(2))) vo
             x = A.r0[traj];
             v = A.v0[traj];
         }
-        double Eprev = -1.0;
+        double Eprev = -1.0, u2prev = 0.0, hprev = 0.0;
         bool warm = false;
         int nh = 0;
 
         // eigen at x (all threads); leaves E, U in LDS and returns the model scalars
         auto eigen = [&](double xx) -> Scalars {
+            IE_IDS
             const Scalars s = na_scalars(A, xx);
             // four lanes per root, roots dealt round-robin over the wavefronts (16 NT >= N slots)
             const int ir = (l >> 2) * NT + w, sub = l & 3;
             if (ir < N) {
                 double fp;
-                const double lam = na_root<4>(eps, M, A.a, V2, zn, s.h, ir, warm, Eprev, fp, sub);
+                // first-order start: dE/dh = u^2 (the impurity entry alone depends on x)
+                const double lam = na_root<4>(eps, M, A.a, V2, zn, s.h, ir, warm, Eprev + (s.h - hprev) * u2prev, Eprev, fp, sub);
+                const double u = 1.0 / sqrt(fp);
                 if (sub == 0) {
                     E[ir] = lam;
-                    U[ir] = 1.0 / sqrt(fp);
+                    U[ir] = u;
                 }
                 Eprev = lam;
+                u2prev = u * u;
             } else if (ir < NP && sub == 0) {
                 E[ir] = 0.0;
                 U[ir] = 0.0;
             }
             warm = true;
+            hprev = s.h;
             __syncthreads();
             return s;
         };
         // eigenpairs at a bead position into Eb, Ub (cold start: no roots are kept per bead)
         auto bead_eigen = [&](double xx) -> Scalars {
+            IE_IDS
             const Scalars s = na_scalars(A, xx);
             const int ir = (l >> 2) * NT + w, sub = l & 3;
             if (ir < N) {
                 double fp;
-                const double lam = na_root<4>(eps, M, A.a, V2, zn, s.h, ir, false, 0.0, fp, sub);
+                const double lam = na_root<4>(eps, M, A.a, V2, zn, s.h, ir, false, 0.0, 0.0, fp, sub);
                 if (sub == 0) {
                     Eb[ir] = lam;
                     Ub[ir] = 1.0 / sqrt(fp);
@@ -461,12 +482,11 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(2))) vo
         // acceleration at the eigenpairs whose impurity components are Uv, with the wavefunction in Tb
         // (iesh.jl:190-207, ehrenfest_na.jl:72-86; per bead rpiesh.jl:20-38, rpehrenfest_na.jl:14-40)
         auto accel = [&](const Scalars& s, const double* Uv) -> double {
+            IE_IDS
+            // summed by every wavefront for itself (Ne <= 64)
+            double t = 0.0;
             if (A.method == 0) {
-                if (tid == 0) {
-                    double f = s.dU0;
-                    for (int e = 0; e < Ne; ++e) { const double u = Uv[occ[e]]; f += u * s.dh * u; }
-                    scal[0] = f;
-                }
+                if (l < Ne) { const double u = Uv[occ[l]]; t = u * s.dh * u; }
             } else {
                 if (tid < Ne) {
                     double re = 0.0, im = 0.0;
@@ -477,22 +497,16 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(2))) vo
                     pcol[tid] = s.dh * (re * re + im * im);
                 }
                 __syncthreads();
-                if (tid == 0) {
-                    double f = s.dU0;
-                    for (int e = 0; e < Ne; ++e) f += pcol[e];
-                    scal[0] = f;
-                }
+                if (l < Ne) t = pcol[l];
             }
-            __syncthreads();
-            const double f = scal[0];
-            __syncthreads();
-            return -f / A.mass;
+            return -(s.dU0 + wave_sum(t)) / A.mass;
         };
         // Diabatic populations: component a of eigenvector b is U_ab = u_b (a = 0, impurity) or
         // V u_b / (E_b - eps_{a-1}) (bath level a - 1).  IESH (iesh.jl:351-369): per electron
         // diag(U rho U^T), rho = offdiag(c c^T) + e_s e_s^T with c = Re psi_e, i.e.
         // (sum_b U_ab c_b)^2 - sum_b U_ab^2 c_b^2 + U_as^2; EhrenfestNA: sum_e |(U psi)_{a e}|^2.
         auto save = [&](int slot) {
+            IE_IDS
             if (slot >= A.nsave) return;
             if (A.method == 0) {
                 for (int b = tid; b < N; b += B) {
@@ -515,7 +529,7 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(2))) vo
 #pragma unroll
                         for (int q = 0; q < 4; ++q) { sr[q] = 0.0; si[q] = 0.0; }
                         for (int b = 0; b < N; ++b) {
-                            const double u = (a == 0) ? U[b] : A.V * U[b] / (E[b] - ea);
+                            const double u = (a == 0) ? U[b] : A.V * U[b] * rcp_nr(E[b] - ea);
                             const double* row = Tb + b * CW + 2 * e0;
 #pragma unroll
                             for (int q = 0; q < 4; ++q) {
@@ -530,12 +544,12 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(2))) vo
                     }
                     if (A.method == 0) {
                         for (int b = sub; b < N; b += 4) {
-                            const double u = (a == 0) ? U[b] : A.V * U[b] / (E[b] - ea);
+                            const double u = (a == 0) ? U[b] : A.V * U[b] * rcp_nr(E[b] - ea);
                             pa -= u * u * pcol[b];
                         }
                         for (int e = sub; e < Ne; e += 4) {
                             const int sb = occ[e];
-                            const double u = (a == 0) ? U[sb] : A.V * U[sb] / (E[sb] - ea);
+                            const double u = (a == 0) ? U[sb] : A.V * U[sb] * rcp_nr(E[sb] - ea);
                             pa += u * u;
                         }
                     }
@@ -560,17 +574,19 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(2))) vo
 
         // bead accelerations into bal (one bead at a time over the whole workgroup)
         auto bead_accels = [&]() {
+            IE_IDS
             for (int b = 0; b < P; ++b) {
                 const Scalars s = bead_eigen(brl[b]);
                 const double a = accel(s, Ub);
                 if (tid == 0) bal[b] = a;
+                __syncthreads();  // Ub and pcol are the next bead's
             }
-            __syncthreads();
         };
         // y = H x for the two bead vectors (H: the discrete Hartley transform, orthogonal and its own
         // inverse; modes l and P - l share the frequency, so the Cayley step per Hartley mode is the
         // free ring polymer's), one bead per lane of wavefront 0
         auto hartley2 = [&](const double* x1, const double* x2, double* y1, double* y2) {
+            IE_IDS
             if (tid < P) {
                 double a1 = 0.0, a2 = 0.0;
                 for (int k = 0; k < P; ++k) {
@@ -591,6 +607,7 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(2))) vo
         if (rp) bead_accels();
         else kacc = accel(sc, U);
         save(0);
+        __syncthreads();
 
         for (int64_t step = 0; step < A.nsteps; ++step) {
             if (!rp) {
@@ -622,31 +639,47 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(2))) vo
                 __syncthreads();
             }
 
+            double dtvd;  // dt sum |v_dot_d[m, n]| over unoccupied m and electrons n (iesh.jl:285-298)
             // ---- wavefunction: psi <- exp(-i dt H) psi, H = diag(E) - i v d ---------------------------
             {
+            IE_IDS
                 const double sW = dt * v * sc.dh;
                 const int ia = 16 * w + (l & 15);
+                const bool free_row = isocc[ia] < 0;
+                const double Ei = E[ia], sU = -sW * U[ia];
                 double Af[KF];
-                double loc = 0.0;
+                double loc = 0.0, lvd = 0.0;
 #pragma unroll
                 for (int kk = 0; kk < KF; ++kk) {
                     const int k = 4 * kk + (l >> 4);
-                    double val = 0.0;
-                    if (ia < N && k < N && ia != k) val = -sW * (U[ia] * U[k] / (E[k] - E[ia]));
+                    double val = sU * (U[k] * rcp_nr(E[k] - Ei));
+                    if (ia >= N || k >= N || ia == k) val = 0.0;
                     Af[kk] = val;
                     loc += val * val;
+                    if (!RPB && free_row && isocc[k] >= 0) lvd += fabs(val);
                 }
-                // ||dt H||_2 <= dt max|E_i| + ||dt v d||_F
-                const double fro = sqrt(block_sum<NT>(loc, red));
-                const double theta = dt * block_max<NT>(tid < N ? fabs(E[tid]) : 0.0, red) + fro;
+                loc = wave_sum(loc);
+                if (!RPB) lvd = wave_sum(lvd);
+                if (l == 0) {
+                    part[w] = loc;
+                    part[8 + w] = lvd;
+                }
+                __syncthreads();
+                loc = part[0];
+                dtvd = part[8];
+#pragma unroll
+                for (int j = 1; j < NT; ++j) {
+                    loc += part[j];
+                    dtvd += part[8 + j];
+                }
+                // ||dt H||_2 <= dt max|E_i| + ||dt v d||_F; the energies ascend
+                const double theta = dt * fmax(fabs(E[0]), fabs(E[N - 1])) + sqrt(loc);
                 // Sub-steps of norm <= 0.5, at most 1024 of them; a non-finite bound leaves psi as is.
                 const bool finite = theta <= 512.0;
-                const int ns = (finite && theta > 0.5) ? (int)ceil(theta / 0.5) : 1;
-                const double ths = finite ? theta / ns : 0.0, eth = exp(ths);
-                int K = 0;
-                double term = 1.0;
-                while (finite && K < 40 && term * ths / (K + 1) * eth > 1e-17) { ++K; term *= ths / K; }
+                const int ns = (finite && theta > 0.5) ? __builtin_amdgcn_readfirstlane((int)ceil(theta / 0.5)) : 1;
                 const double inv_ns = 1.0 / ns;
+                const double ths = finite ? theta * inv_ns : 0.0;
+                const int K = (int)__popcll(__ballot((float)ths > order_from));
                 if (ns > 1) {
 #pragma unroll
                     for (int kk = 0; kk < KF; ++kk) Af[kk] *= inv_ns;
@@ -655,46 +688,65 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(2))) vo
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int ir = 16 * w + 4 * r + (l >> 4);
-                    dg[r] = (ir < N) ? dt * E[ir] * inv_ns : 0.0;
+                    // the sign of the Re / Im column this lane holds goes with it
+                    dg[r] = (ir < N) ? ((l & 1) ? -dt : dt) * E[ir] * inv_ns : 0.0;
                 }
                 d4 P[CTM];
+                const int own = (16 * w + (l >> 4)) * CW + (l & 15);
 #pragma unroll
                 for (int ct = 0; ct < CTM; ++ct) {
+                    P[ct] = d4{0.0, 0.0, 0.0, 0.0};
                     if (ct < CT) {
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) P[ct][r] = Tb[(16 * w + 4 * r + (l >> 4)) * CW + 16 * ct + (l & 15)];
+                        for (int r = 0; r < 4; ++r) P[ct][r] = Tb[own + 4 * r * CW + 16 * ct];
                     }
                 }
-                // Column tiles are independent in the GEMM: each tile of the next term is computed,
-                // then written back over the same tile after every wave has read it.
+                // All column tiles of a term are computed, then written back over it: two barriers a term.
                 const double* bcol = Tb + (l >> 4) * CW + (l & 15);
-                for (int sub = 0; sub < ns; ++sub) {
+                for (int sub = 0; sub < ns && K > 0; ++sub) {
                     for (int k = 1; k <= K; ++k) {
-                        const double ik = 1.0 / k;
+                        const double ik = rcp_nr((double)k);
                         const bool last = (k == K);
+                        d4 Y[CTM];
 #pragma unroll
                         for (int ct = 0; ct < CTM; ++ct) {
                             if (ct < CT) {
-                                d4 Y = d4{0.0, 0.0, 0.0, 0.0};
+                                Y[ct] = d4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-                                for (int kk = 0; kk < KF; ++kk)
-                                    Y = __builtin_amdgcn_mfma_f64_16x16x4f64(Af[kk], bcol[4 * kk * CW + 16 * ct], Y, 0, 0, 0);
-                                const int j = 16 * ct + (l & 15);
+                                for (int kk = 0; kk < KF; ++kk) {
+                                    if (kk > KF - 4 && 4 * kk >= N) continue;  // padding
+                                    Y[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(Af[kk], bcol[4 * kk * CW + 16 * ct], Y[ct], 0, 0, 0);
+                                }
 #pragma unroll
                                 for (int r = 0; r < 4; ++r) {
-                                    const double part = Tb[(16 * w + 4 * r + (l >> 4)) * CW + (j ^ 1)];
-                                    Y[r] = (Y[r] + ((j & 1) ? -dg[r] : dg[r]) * part) * ik;
-                                    P[ct][r] += Y[r];
+                                    Y[ct][r] = (Y[ct][r] + dg[r] * Tb[(own ^ 1) + 4 * r * CW + 16 * ct]) * ik;
+                                    P[ct][r] += Y[ct][r];
                                 }
-                                __syncthreads();
-#pragma unroll
-                                for (int r = 0; r < 4; ++r) Tb[(16 * w + 4 * r + (l >> 4)) * CW + j] = last ? P[ct][r] : Y[r];
                             }
                         }
                         __syncthreads();
+#pragma unroll
+                        for (int ct = 0; ct < CTM; ++ct) {
+                            if (ct < CT) {
+#pragma unroll
+                                for (int r = 0; r < 4; ++r) Tb[own + 4 * r * CW + 16 * ct] = last ? P[ct][r] : Y[ct][r];
+                            }
+                        }
+                        if (sub + 1 < ns || !last) __syncthreads();
                     }
-                    if (K == 0) break;
                 }
+                // the weight of the orbitals outside the occupied states
+                double lt2 = 0.0;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    double q = 0.0;
+#pragma unroll
+                    for (int ct = 0; ct < CTM; ++ct) q += P[ct][r] * P[ct][r];
+                    if (isocc[16 * w + 4 * r + (l >> 4)] < 0) lt2 += q;
+                }
+                lt2 = wave_sum(lt2);
+                if (l == 0) part[16 + w] = lt2;
+                __syncthreads();
             }
 
             if (rp) {  // centroid at the step end: eigenpairs and velocity for the hop and the next step
@@ -709,26 +761,35 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(2))) vo
 
             // ---- IESH hop (iesh.jl:390-407) -------------------------------------------------------------
             if (A.method == 0) {
+            IE_IDS
                 const double rnd = philox_uniform((uint64_t)traj, (uint32_t)step, STREAM_HOP, A.key);
                 const int LD = Ne | 1, Nu = N - Ne;
                 double* Sre = Sb;
                 double* Sim = Sb + Ne * LD;
-                // sum |v_dot_d[m, n]| over unoccupied m and electrons n (iesh.jl:285-298), and
-                // t2 = ||psi[unoccupied, :]||_F^2, the weight of the orbitals outside the occupied rows
-                double lvd = 0.0, lt2 = 0.0;
-                for (int k = tid; k < N * Ne; k += B) {
-                    const int m = k / Ne, n = k - m * Ne;
-                    if (isocc[m] < 0) {
-                        const int o = occ[n];
-                        lvd += fabs(v * (sc.dh * (U[m] * U[o] / (E[o] - E[m]))));
-                        const double pr = Tb[m * CW + 2 * n], pi = Tb[m * CW + 2 * n + 1];
-                        lt2 += pr * pr + pi * pi;
+                // t2 = ||psi[unoccupied, :]||_F^2, the weight of the orbitals outside the occupied rows; a ring
+                // polymer's eigenpairs and velocity are those of the step end
+                double t2 = part[16];
+#pragma unroll
+                for (int j = 1; j < NT; ++j) t2 += part[16 + j];
+                if (RPB) {
+                    double lvd = 0.0;
+                    for (int k = tid; k < N * Ne; k += B) {
+                        const int m = k / Ne, n = k - m * Ne;
+                        if (isocc[m] < 0) {
+                            const int o = occ[n];
+                            lvd += fabs(v * (sc.dh * (U[m] * U[o] / (E[o] - E[m]))));
+                        }
                     }
+                    lvd = wave_sum(lvd);
+                    if (l == 0) part[24 + w] = lvd;
+                    __syncthreads();
+                    dtvd = part[24];
+#pragma unroll
+                    for (int j = 1; j < NT; ++j) dtvd += part[24 + j];
+                    dtvd *= dt;
                 }
-                const double sumvd = block_sum<NT>(lvd, red);
-                const double t2 = block_sum<NT>(lt2, red);
-                // The estimate 2 dt sumvd (|Re det S| + |Im det S|) / |det S|^2 (iesh.jl:250-253) is at
-                // most 2 dt sumvd sqrt(2) / |det S|, and for orthonormal orbitals (S^H S + T^H T = I,
+                // The estimate 2 dtvd (|Re det S| + |Im det S|) / |det S|^2 (iesh.jl:250-253) is at
+                // most 2 dtvd sqrt(2) / |det S|, and for orthonormal orbitals (S^H S + T^H T = I,
                 // T = psi[unoccupied, :]) |det S|^2 = prod(1 - s_i^2(T)) >= 1 - t2.  Where that bound
                 // is already below the uniform, the reference's estimate is too: no hop, and the LU is
                 // skipped (1e-6 absorbs the orbitals' rounding-level loss of orthonormality; 1e-8 and
@@ -736,20 +797,24 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(2))) vo
                 bool skip = false;
                 if (det_bound) {
                     const double L2 = 1.0 - t2 - 1e-6;
-                    skip = L2 > 1e-4 && 2.0 * dt * sumvd * 1.4142135623730951 * (1.0 + 1e-8) < rnd * sqrt(L2);
+                    skip = L2 > 1e-4 && 2.0 * dtvd * 1.4142135623730951 * (1.0 + 1e-8) < rnd * sqrt(L2);
                 }
                 bool evaluate = false;
                 if (!skip) {
+                    IE_IDS
                     // S_je = psi[occ_j, e] (iesh.jl:309-316) as real / imaginary planes, row stride LD (odd)
                     for (int idx = tid; idx < Ne * Ne; idx += B) {
                         const int j = idx / Ne, e = idx - j * Ne;
                         Sre[j * LD + e] = Tb[occ[j] * CW + 2 * e];
                         Sim[j * LD + e] = Tb[occ[j] * CW + 2 * e + 1];
                     }
-                    if (tid == 0) {  // unoccupied states in ascending order (DynamicsUtils.jl:162-171)
+                    if (w == 0) {  // unoccupied states in ascending order (DynamicsUtils.jl:162-171)
                         int c = 0;
-                        for (int m = 0; m < N; ++m)
-                            if (isocc[m] < 0) unocc[c++] = m;
+                        for (int m = l; m - l < N; m += 64) {
+                            const uint64_t f = __ballot(m < N && isocc[min(m, N - 1)] < 0);
+                            if ((f >> l) & 1) unocc[c + __popcll(f & ((1ull << l) - 1))] = m;
+                            c += __popcll(f);
+                        }
                     }
                     __syncthreads();
                     // det S (FastDeterminant.jl:20-22) on wavefront 0
@@ -766,11 +831,11 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(2))) vo
                     const double dre = scal[1], dim = scal[2];
                     const bool singular = scal[3] != 0.0;
                     const double Akk = dre * dre + dim * dim;
-                    const double pref = 2.0 * dt / Akk;
-                    const double est = pref * sumvd * (fabs(dre) + fabs(dim));
+                    const double est = 2.0 / Akk * dtvd * (fabs(dre) + fabs(dim));
                     evaluate = !singular && Akk > 0.0 && (!A.estimate || !(est < rnd));
                 }
                 if (evaluate) {
+                    IE_IDS
                     __syncthreads();  // wavefront 0's determinant work on Sb is complete
                     for (int idx = tid; idx < Ne * Ne; idx += B) {
                         const int j = idx / Ne, e = idx - j * Ne;
@@ -951,6 +1016,7 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(2))) vo
                 }
                 // ---- Granucci-Persico EDC per electron (decoherence_corrections.jl:21-39, iesh.jl:424-433)
                 if (A.edc) {
+                    IE_IDS
                     const double Ekin = 0.5 * A.mass * v * v;
                     if (tid < Ne) {
                         const int s = occ[tid];
@@ -1040,7 +1106,7 @@ __global__ __launch_bounds__(256) void ie_initial_energies(const IeshArgs A, int
     double* row = W + traj * (diabatic ? 3 * A.N : A.N);
     for (int ir = threadIdx.x & 63; ir < A.N; ir += 64) {
         double fp;
-        const double lam = na_root(eps, A.M, A.a, A.V * A.V, zn, s.h, ir, false, 0.0, fp);
+        const double lam = na_root(eps, A.M, A.a, A.V * A.V, zn, s.h, ir, false, 0.0, 0.0, fp);
         if (diabatic) {
             row[ir] = (ir == 0) ? s.h : eps[ir - 1];
             row[A.N + ir] = lam;
