@@ -21,8 +21,8 @@
 //     (-dt v dh W) [Re psi | Im psi] on FP64 MFMA 16x16x4 plus the diagonal part.  The reference
 //     diagonalises H with zheevr and forms U exp(-i Lambda dt) U^H; both give exp(-i H dt) to
 //     rounding.
-//   * IESH hop: S = psi[occ, :], det S by LU (partial pivoting) on one wavefront, the reference's
-//     early-exit estimate, and on the (rare) steps that pass it the replaced-row determinants by the
+//   * IESH hop: S = psi[occ, :], det S and S^-1 by one Gauss-Jordan elimination (partial pivoting) in
+//     registers, the reference's early-exit estimate, and on the steps that pass it the replaced-row determinants by the
 //     determinant lemma det(S with row n <- psi_m) = det(S) (psi_m S^-1)_n, so
 //     P(n -> m) = 2 dt Re((psi_m S^-1)_n) v_dot_d[m, n]; cumulative selection electrons outer,
 //     unoccupied states inner (iesh.jl:318-335).
@@ -44,6 +44,7 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 
 constexpr int kIeMaxNe = 64;
 constexpr int kIeMaxStates = 128;
+constexpr double kFarPole = 1e300;  // pads the bath levels to a multiple of 16: nothing in the secular sums
 constexpr size_t kIeLdsBytes = 160 * 1024;  // LDS of one gfx950 compute unit
 
 struct IeshArgs {
@@ -136,16 +137,18 @@ __device__ double secular_root(const double* eps, int M, int i, double V2, doubl
     double lam = (guess > lo && guess < hi) ? guess : 0.5 * (lo + hi);
     fp = 1.0;
     for (int it = 0; it < 100; ++it) {
-        // q_k > 0 below the interval, < 0 above it
+        // q_k > 0 below the interval, < 0 above it; four poles at a time (eps is padded with far poles)
         double sl = 0.0, sl2 = 0.0, sh = 0.0, sh2 = 0.0;
-        for (int k = sub; k < M; k += G) {
-            const double q = rcp_nr(lam - eps[k]);
-            const double q2 = q * q;
-            const bool below = k < i;
-            sl += below ? q : 0.0;
-            sh += below ? 0.0 : q;
-            sl2 += below ? q2 : 0.0;
-            sh2 += below ? 0.0 : q2;
+        for (int k = sub; k < M; k += 4 * G) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const double q = rcp_nr(lam - eps[k + u * G]);
+                const double ql = fmax(q, 0.0), qh = fmin(q, 0.0);
+                sl += ql;
+                sh += qh;
+                sl2 = fma(ql, ql, sl2);
+                sh2 = fma(qh, qh, sh2);
+            }
         }
         if (G > 1) {
             sl = group_sum<G>(sl);
@@ -189,24 +192,20 @@ __device__ __forceinline__ double readlane_f64(double x, int lane) {
     return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
 
-// Sum over the wavefront, the same value in every lane: butterflies inside each row of 16 lanes, then the four rows.
-__device__ __forceinline__ double wave_sum(double v) {
+// Sums over rows of 16 lanes and over the wavefront, the same value in every lane: butterflies inside the rows, then
+// the four rows.
+__device__ __forceinline__ double row_sum(double v) {
     v += dpp_f64<0xB1>(v);
     v += dpp_f64<0x4E>(v);
     v += dpp_f64<0x141>(v);  // row_half_mirror
     v += dpp_f64<0x140>(v);  // row_mirror
+    return v;
+}
+__device__ __forceinline__ double wave_sum(double v) {
+    v = row_sum(v);
     return (readlane_f64(v, 0) + readlane_f64(v, 16)) + (readlane_f64(v, 32) + readlane_f64(v, 48));
 }
 
-// Orders this wavefront's LDS accesses: its lanes exchange data through LDS without a workgroup
-// barrier (a wavefront's LDS instructions execute in program order).
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
-// One step of a wavefront arg-max over (mag, idx) with the DPP lane pattern CTRL (larger mag
-// wins, the lower idx on ties).
 // Eigenvalue ir of the Newns-Anderson matrix at impurity energy h: the secular root on its
 // bracket (the outer brackets reach past the band and h by the coupling norm zn = sqrt(M) V);
 // warm starts from `guess` (from `prev` where that leaves the bracket), a cold start from below the bracket.
@@ -221,6 +220,8 @@ __device__ __forceinline__ double na_root(const double* eps, int M, double a, do
                            4.0e-16 * scale, fp, sub);
 }
 
+// One step of a wavefront arg-max over (mag, idx) with the DPP lane pattern CTRL (larger mag
+// wins, the lower idx on ties).
 template <int CTRL>
 __device__ __forceinline__ void argmax_dpp(double& mag, int& idx) {
     const long long bits = __double_as_longlong(mag);
@@ -251,64 +252,70 @@ __device__ __forceinline__ void wave_argmax(double& mag, int& idx) {
     idx = bi;
 }
 
-// det of the Ne x Ne complex matrix held as real / imaginary planes with row stride LD, by LU with
-// partial pivoting (largest |.| in the column, lowest row on ties) on one wavefront: lane r holds
-// row r, rows are eliminated in place and never moved, and the sign of the pivot permutation
-// comes from counting, at each step, the remaining rows above the pivot row.  Each lane keeps the
-// current column of its row in registers; the rest of the row is updated through LDS in chunks of
-// eight columns whose loads are all issued before its stores.  The matrix is overwritten.
-// Returns false for a singular matrix (a zero pivot column).  Called by all 64 lanes.
-__device__ bool wave_det(double* Sre, double* Sim, int LD, int Ne, double& dre, double& dim) {
-    constexpr int kChunk = 8;
-    const int r = __lane_id();
-    bool used = r >= Ne;
-    double cr = used ? 0.0 : Sre[r * LD], ci = used ? 0.0 : Sim[r * LD];  // S[r][p]
+// Inverse and determinant of an Ne x Ne complex matrix (Ne <= 64) by Gauss-Jordan elimination in place with partial
+// pivoting (largest |.| in the column among the rows not yet used, lowest row on ties), by NT wavefronts: lane r holds
+// row r, wavefront w the columns w, w + NT, ..., rotated so that its next pivot column is always x[0].  Rows are never
+// moved: with row q_p the pivot row of column p, entry (p, q_c) of the inverse ends in row q_p, column c, and the sign
+// of the pivot permutation comes from counting, at each step, the unused rows above the pivot row.  The column's owner
+// picks the pivot and leaves the multipliers in LDS; one barrier a pivot (two buffers), everything else in registers.
+// One wavefront's LU through LDS followed by a workgroup's Gauss-Jordan through LDS took 116 us at 20 electrons and
+// 290 us at 50.  buf: 2 x 136 doubles; piv[p] = q_p; myp: the column whose pivot row this lane's row was; on return
+// x[j] is column w + NT ((j + rot) % KC).  False for a singular matrix (a zero pivot column).  Called by whole
+// workgroups of 64 NT lanes; the caller's previous use of buf and piv ends with a barrier.
+template <int NT, int KC>
+__device__ __forceinline__ bool block_inverse(double (&xr)[KC], double (&xi)[KC], int Ne, int w, int l, double* buf, int* piv,
+                                              double& dre, double& dim, int& myp, int& rot) {
+    bool used = l >= Ne;
     double ar = 1.0, ai = 0.0;
-    int inv = 0;
+    int inv = 0, owner = 0;
+    myp = 0;
+    rot = 0;
     for (int p = 0; p < Ne; ++p) {
-        double mag = used ? -1.0 : cr * cr + ci * ci;
-        int idx = r;
-        wave_argmax(mag, idx);
-        if (!(mag > 0.0)) { dre = 0.0; dim = 0.0; return false; }
-        const int q = idx;
-        inv += __popcll(__ballot(!used && r < q));
-        const double pr = readlane_f64(cr, q), pi = readlane_f64(ci, q);
+        double* B = buf + (p & 1) * 136;
+        if (w == owner) {
+            double mag = used ? -1.0 : xr[0] * xr[0] + xi[0] * xi[0];
+            int q = l;
+            wave_argmax(mag, q);
+            const bool ok = mag > 0.0;
+            const double pr = readlane_f64(xr[0], q), pi = readlane_f64(xi[0], q), ip = 1.0 / mag;
+            B[2 * l] = (xr[0] * pr + xi[0] * pi) * ip;      // S[r][p] / pivot
+            B[2 * l + 1] = (xi[0] * pr - xr[0] * pi) * ip;
+            if (l == 0) {
+                B[128] = pr;
+                B[129] = pi;
+                B[130] = pr * ip;                           // 1 / pivot
+                B[131] = -pi * ip;
+                piv[p] = ok ? q : -1;
+            }
+        }
+        __syncthreads();
+        const int q = __builtin_amdgcn_readfirstlane(piv[p]);
+        if (q < 0) { dre = 0.0; dim = 0.0; return false; }
+        const double pr = B[128], pi = B[129];
+        const double fr = l == q ? -B[130] : B[2 * l], fi = l == q ? -B[131] : B[2 * l + 1];
         {
             const double nr = ar * pr - ai * pi, ni = ar * pi + ai * pr;
             ar = nr;
             ai = ni;
         }
-        if (r == q) used = true;
-        wave_lds_sync();  // the pivot row's stores of the previous step are visible
-        if (!used) {
-            const double ip = 1.0 / mag;
-            const double fr = (cr * pr + ci * pi) * ip, fi = (ci * pr - cr * pi) * ip;  // S[r][p] / pivot
-            for (int c0 = p + 1; c0 < Ne; c0 += kChunk) {
-                double yr[kChunk], yi[kChunk], xr[kChunk], xi[kChunk];
+        inv += __popcll(__ballot(!used && l < q));
+        if (l == q) { used = true; myp = p; }
 #pragma unroll
-                for (int k = 0; k < kChunk; ++k) {
-                    const int c = c0 + k < Ne ? c0 + k : Ne - 1;
-                    yr[k] = Sre[q * LD + c];
-                    yi[k] = Sim[q * LD + c];
-                    xr[k] = Sre[r * LD + c];
-                    xi[k] = Sim[r * LD + c];
-                }
-#pragma unroll
-                for (int k = 0; k < kChunk; ++k) {
-                    xr[k] -= fr * yr[k] - fi * yi[k];
-                    xi[k] -= fr * yi[k] + fi * yr[k];
-                }
-                if (c0 == p + 1) { cr = xr[0]; ci = xi[0]; }
-#pragma unroll
-                for (int k = 0; k < kChunk; ++k) {
-                    if (c0 + k < Ne) {
-                        Sre[r * LD + c0 + k] = xr[k];
-                        Sim[r * LD + c0 + k] = xi[k];
-                    }
-                }
-            }
+        for (int j = 0; j < KC; ++j) {  // rows r != q: x - f y; row q: y / pivot
+            const double yr = readlane_f64(xr[j], q), yi = readlane_f64(xi[j], q);
+            const double zr = l == q ? 0.0 : xr[j], zi = l == q ? 0.0 : xi[j];
+            xr[j] = fma(fi, yi, fma(-fr, yr, zr));
+            xi[j] = fma(-fi, yr, fma(-fr, yi, zi));
         }
-        wave_lds_sync();
+        if (w == owner) {  // the pivot column's own place takes the identity's column; then the next one to the front
+            const double tr = -fr, ti = -fi;
+#pragma unroll
+            for (int j = 0; j + 1 < KC; ++j) { xr[j] = xr[j + 1]; xi[j] = xi[j + 1]; }
+            xr[KC - 1] = tr;
+            xi[KC - 1] = ti;
+            ++rot;
+        }
+        if (++owner == NT) owner = 0;
     }
     dre = (inv & 1) ? -ar : ar;
     dim = (inv & 1) ? -ai : ai;
@@ -331,12 +338,13 @@ __device__ __forceinline__ int ie_tid() {
 }
 #define IE_IDS const int tid = ie_tid(), w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63; (void)w; (void)l;
 
-// Bound by the matrix cores in the propagator (8 or 9 terms of N x N x 2 Ne) and, up to 64 states, by the latency of
-// the phases around it, which one workgroup cannot hide: there the registers are held to three wavefronts a SIMD, so
-// that three or four trajectories share a compute unit (those phases were 41 of a step's 57 us at 41 states).  Larger problems fill the LDS with one trajectory and keep two wavefronts' registers.  The phases
-// exchange sums once (coupling norm, hop bound, orbital weight ride on the propagator's registers and barriers) and
-// divide by Newton-Raphson reciprocals.  8192 trajectories of 41 states, 100 steps: 92.3 -> 65.9 ms; 2048 of 101
-// states, 50 steps: 102.5 -> 95.5 ms.
+// Bound by the matrix cores in the propagator (8 or 9 terms of N x N x 2 Ne; 109 of a step's 140 us at 101 states, where
+// seven wavefronts share four SIMDs) and, up to 64 states, by the latency of the phases around it, which one workgroup
+// cannot hide: there the registers are held to three wavefronts a SIMD, so that three or four trajectories share a
+// compute unit.  Larger problems fill the LDS with one trajectory and keep two wavefronts' registers.  The phases
+// exchange sums once (coupling norm, hop bound, orbital weight ride on the propagator's registers and barriers),
+// divide by Newton-Raphson reciprocals, save populations by a product on the matrix cores and invert S in registers.
+// 8192 trajectories of 41 states, 100 steps: 91 -> 56 ms; 2048 of 101 states, 50 steps: 103 -> 66 ms.
 // RPB: ring polymer (BCBWavefunction), a separate instantiation so the one-bead kernels carry none of it
 template <int NT, int CTM, bool RPB>
 __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(NT <= 4 && CTM <= 4 && !RPB ? 3 : 2))) void iesh_kernel(const IeshArgs A) {
@@ -347,7 +355,7 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(NT <= 4
     constexpr int CW = 16 * CTM; // row stride of psi in LDS (compile time, so LDS offsets are immediates)
     const int N = A.N, M = A.M, Ne = A.Ne, CT = A.cw / 16;
     double* Tb = smem;                       // NP x CW: psi (Re, Im interleaved per electron) / Taylor term
-    double* Sb = Tb + NP * CW;               // Ne x Ne complex S, inverted in place
+    double* Sb = Tb + NP * CW;               // Ne x Ne complex S^-1
     double* E = Sb + A.sb_len;               // NP adiabatic energies
     double* U = E + NP;                      // NP impurity components of the eigenvectors
     double* eps = U + NP;                    // NP bath levels
@@ -374,7 +382,7 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(NT <= 4
     const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
     const double dt = A.dt;
     const double V2 = A.V * A.V;
-    for (int k = tid; k < NP; k += B) eps[k] = (k < M) ? A.a + k * A.de : 0.0;
+    for (int k = tid; k < NP; k += B) eps[k] = (k < M) ? A.a + k * A.de : kFarPole;
     __syncthreads();
     const double zn = sqrt((double)M) * A.V;
     const float order_from = (threadIdx.x & 63) < 16 ? kTaylorFrom[threadIdx.x & 15] : __builtin_inff();
@@ -508,65 +516,59 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(NT <= 4
         auto save = [&](int slot) {
             IE_IDS
             if (slot >= A.nsave) return;
-            if (A.method == 0) {
-                for (int b = tid; b < N; b += B) {
-                    double wb = 0.0;
-                    for (int e = 0; e < Ne; ++e) { const double c = Tb[b * CW + 2 * e]; wb += c * c; }
-                    pcol[b] = wb;
+            // U psi on the matrix cores, as a term of the propagator; IESH takes the real columns and puts the rest,
+            // sum_b U_ab^2 ([b occupied] - sum_e c_b^2), in weights
+            const int g = l >> 4, own = (16 * w + g) * CW + (l & 15);
+            const bool drop = A.method == 0 && (l & 1);
+            double rs[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                double q = 0.0;
+                for (int ct = 0; ct < CT; ++ct) { const double c = Tb[own + 4 * r * CW + 16 * ct]; q += c * c; }
+                rs[r] = row_sum(drop ? 0.0 : q);
+                if ((l & 15) == 0) {
+                    const int b = 16 * w + 4 * r + g;
+                    pcol[b] = (isocc[b] >= 0 ? 1.0 : 0.0) - rs[r];
                 }
-                __syncthreads();
             }
-            // four lanes per diabatic state a (4 N <= 64 NT lanes): lane sub takes the 4-electron
-            // chunks sub, sub + 4, ... and every fourth term of the IESH corrections; the quad's
-            // partial sums are combined by DPP (same bits in all four lanes)
+            __syncthreads();
             {
-                const int a = tid >> 2, sub = tid & 3;
-                double pa = 0.0;
-                if (a < N) {
-                    const double ea = (a == 0) ? 0.0 : eps[a - 1];
-                    for (int e0 = 4 * sub; e0 < Ne; e0 += 16) {
-                        double sr[4], si[4];
+                const int a = 16 * w + (l & 15);
+                const double ea = (a > 0 && a < N) ? eps[a - 1] : 0.0;
+                double Af[KF], corr = 0.0;
 #pragma unroll
-                        for (int q = 0; q < 4; ++q) { sr[q] = 0.0; si[q] = 0.0; }
-                        for (int b = 0; b < N; ++b) {
-                            const double u = (a == 0) ? U[b] : A.V * U[b] * rcp_nr(E[b] - ea);
-                            const double* row = Tb + b * CW + 2 * e0;
-#pragma unroll
-                            for (int q = 0; q < 4; ++q) {
-                                if (e0 + q < Ne) {
-                                    sr[q] += u * row[2 * q];
-                                    if (A.method != 0) si[q] += u * row[2 * q + 1];
-                                }
-                            }
-                        }
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) pa += sr[q] * sr[q] + si[q] * si[q];
-                    }
-                    if (A.method == 0) {
-                        for (int b = sub; b < N; b += 4) {
-                            const double u = (a == 0) ? U[b] : A.V * U[b] * rcp_nr(E[b] - ea);
-                            pa -= u * u * pcol[b];
-                        }
-                        for (int e = sub; e < Ne; e += 4) {
-                            const int sb = occ[e];
-                            const double u = (a == 0) ? U[sb] : A.V * U[sb] * rcp_nr(E[sb] - ea);
-                            pa += u * u;
-                        }
-                    }
+                for (int kk = 0; kk < KF; ++kk) {
+                    const int k = 4 * kk + g;
+                    double u = (a == 0) ? U[k] : A.V * U[k] * rcp_nr(E[k] - ea);
+                    if (a >= N || k >= N) u = 0.0;
+                    Af[kk] = u;
+                    corr += u * u * pcol[k];
                 }
-                pa = group_sum<4>(pa);
-                if (a < N && sub == 0) {
-                    A.save_di[((size_t)slot * N + a) * A.ntraj + traj] = pa;
-                    double pad;
-                    if (A.method == 0) pad = isocc[a] >= 0 ? 1.0 : 0.0;  // one-hot (iesh.jl:371-375)
-                    else {                                                // ehrenfest_na.jl:119-126
-                        pad = 0.0;
-                        for (int e = 0; e < Ne; ++e) {
-                            const double re = Tb[a * CW + 2 * e], im = Tb[a * CW + 2 * e + 1];
-                            pad += re * re + im * im;
-                        }
+                corr += __shfl_xor(corr, 16);
+                corr += __shfl_xor(corr, 32);
+                double pa[4] = {0.0, 0.0, 0.0, 0.0};
+                const double* bcol = Tb + g * CW + (l & 15);
+                for (int ct = 0; ct < CT; ++ct) {
+                    d4 Y = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                    for (int kk = 0; kk < KF; ++kk) {
+                        if (kk > KF - 4 && 4 * kk >= N) continue;  // padding
+                        Y = __builtin_amdgcn_mfma_f64_16x16x4f64(Af[kk], bcol[4 * kk * CW + 16 * ct], Y, 0, 0, 0);
                     }
-                    A.save_ad[((size_t)slot * N + a) * A.ntraj + traj] = pad;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) pa[r] += Y[r] * Y[r];
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int b = 16 * w + 4 * r + g;
+                    double pd = row_sum(drop ? 0.0 : pa[r]);
+                    const double cb = __shfl(corr, 4 * r + g);
+                    if (A.method == 0) pd += cb;
+                    if ((l & 15) == 0 && b < N) {
+                        A.save_di[((size_t)slot * N + b) * A.ntraj + traj] = pd;
+                        // one-hot (iesh.jl:371-375); ehrenfest_na.jl:119-126
+                        A.save_ad[((size_t)slot * N + b) * A.ntraj + traj] = A.method == 0 ? (isocc[b] >= 0 ? 1.0 : 0.0) : rs[r];
+                    }
                 }
             }
             __syncthreads();
@@ -763,9 +765,7 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(NT <= 4
             if (A.method == 0) {
             IE_IDS
                 const double rnd = philox_uniform((uint64_t)traj, (uint32_t)step, STREAM_HOP, A.key);
-                const int LD = Ne | 1, Nu = N - Ne;
-                double* Sre = Sb;
-                double* Sim = Sb + Ne * LD;
+                const int Nu = N - Ne;
                 // t2 = ||psi[unoccupied, :]||_F^2, the weight of the orbitals outside the occupied rows; a ring
                 // polymer's eigenpairs and velocity are those of the step end
                 double t2 = part[16];
@@ -802,12 +802,6 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(NT <= 4
                 bool evaluate = false;
                 if (!skip) {
                     IE_IDS
-                    // S_je = psi[occ_j, e] (iesh.jl:309-316) as real / imaginary planes, row stride LD (odd)
-                    for (int idx = tid; idx < Ne * Ne; idx += B) {
-                        const int j = idx / Ne, e = idx - j * Ne;
-                        Sre[j * LD + e] = Tb[occ[j] * CW + 2 * e];
-                        Sim[j * LD + e] = Tb[occ[j] * CW + 2 * e + 1];
-                    }
                     if (w == 0) {  // unoccupied states in ascending order (DynamicsUtils.jl:162-171)
                         int c = 0;
                         for (int m = l; m - l < N; m += 64) {
@@ -816,102 +810,38 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(NT <= 4
                             c += __popcll(f);
                         }
                     }
-                    __syncthreads();
-                    // det S (FastDeterminant.jl:20-22) on wavefront 0
-                    if (w == 0) {
-                        double dr, di;
-                        const bool ok = wave_det(Sre, Sim, LD, Ne, dr, di);
-                        if (l == 0) {
-                            scal[1] = dr;
-                            scal[2] = di;
-                            scal[3] = ok ? 0.0 : 1.0;
-                        }
+                    // S_je = psi[occ_j, e] (iesh.jl:309-316): row j on lane j; det S (FastDeterminant.jl:20-22) and S^-1
+                    constexpr int KC = CTM > NT ? 16 : 8;  // columns of a wavefront: 2 Ne <= 16 CTM, Ne <= N <= 16 NT
+                    double xr[KC], xi[KC];
+                    const double* srow = Tb + occ[min(l, Ne - 1)] * CW;
+#pragma unroll
+                    for (int j = 0; j < KC; ++j) {
+                        const int c = w + NT * j;
+                        const bool in = l < Ne && c < Ne;
+                        xr[j] = in ? srow[2 * c] : 0.0;
+                        xi[j] = in ? srow[2 * c + 1] : 0.0;
                     }
-                    __syncthreads();
-                    const double dre = scal[1], dim = scal[2];
-                    const bool singular = scal[3] != 0.0;
+                    double dre, dim;
+                    int myp, rot;
+                    const bool singular = !block_inverse<NT, KC>(xr, xi, Ne, w, l, part + 32, piv, dre, dim, myp, rot);
                     const double Akk = dre * dre + dim * dim;
                     const double est = 2.0 / Akk * dtvd * (fabs(dre) + fabs(dim));
                     evaluate = !singular && Akk > 0.0 && (!A.estimate || !(est < rnd));
+                    if (evaluate && l < Ne) {  // S^-1, interleaved complex, row-major
+#pragma unroll
+                        for (int j = 0; j < KC; ++j) {
+                            const int c = w + NT * ((j + rot) % KC);
+                            if (c < Ne) {
+                                const int at = 2 * (myp * Ne + piv[c]);
+                                Sb[at] = xr[j];
+                                Sb[at + 1] = xi[j];
+                            }
+                        }
+                    }
                 }
                 if (evaluate) {
                     IE_IDS
-                    __syncthreads();  // wavefront 0's determinant work on Sb is complete
-                    for (int idx = tid; idx < Ne * Ne; idx += B) {
-                        const int j = idx / Ne, e = idx - j * Ne;
-                        Sb[2 * idx] = Tb[occ[j] * CW + 2 * e];
-                        Sb[2 * idx + 1] = Tb[occ[j] * CW + 2 * e + 1];
-                    }
-                    // S^-1: Gauss-Jordan inversion of S (interleaved complex, row-major) in place with partial pivoting
-                    bool gj_singular = false;
-                    for (int p = 0; p < Ne; ++p) {
-                        __syncthreads();
-                        if (w == 0) {
-                            double val = -1.0;
-                            int idx = l;
-                            if (l >= p && l < Ne) val = hypot(Sb[2 * (l * Ne + p)], Sb[2 * (l * Ne + p) + 1]);
-#pragma unroll
-                            for (int o = 32; o > 0; o >>= 1) {
-                                const double ov = __shfl_xor(val, o);
-                                const int oi = __shfl_xor(idx, o);
-                                if (ov > val || (ov == val && oi < idx)) { val = ov; idx = oi; }
-                            }
-                            if (l == 0) {
-                                piv[p] = (val > 0.0) ? idx : -1;
-                                scal[1] = Sb[2 * (idx * Ne + p)];
-                                scal[2] = Sb[2 * (idx * Ne + p) + 1];
-                                scal[3] = Sb[2 * (p * Ne + p)];  // moves to row idx with the interchange
-                                scal[4] = Sb[2 * (p * Ne + p) + 1];
-                            }
-                        }
-                        __syncthreads();
-                        const int q = piv[p];
-                        if (q < 0) { gj_singular = true; break; }
-                        const double pr = scal[1], pi = scal[2];
-                        const double den = pr * pr + pi * pi;
-                        const double ir = pr / den, ii = -pi / den;  // 1 / pivot
-                        // column p after the row swap, for the elimination
-                        for (int r = tid; r < Ne; r += B) {
-                            if (r == p) continue;
-                            pcol[2 * r] = (r == q) ? scal[3] : Sb[2 * (r * Ne + p)];
-                            pcol[2 * r + 1] = (r == q) ? scal[4] : Sb[2 * (r * Ne + p) + 1];
-                        }
-                        // swap rows p and q, then scale the pivot row (its pivot entry becomes 1 / pivot)
-                        for (int c = tid; c < Ne; c += B) {
-                            const double ar = Sb[2 * (p * Ne + c)], ai = Sb[2 * (p * Ne + c) + 1];
-                            double br = Sb[2 * (q * Ne + c)], bi = Sb[2 * (q * Ne + c) + 1];
-                            if (q != p) { Sb[2 * (q * Ne + c)] = ar; Sb[2 * (q * Ne + c) + 1] = ai; }
-                            if (c == p) { br = 1.0; bi = 0.0; }
-                            Sb[2 * (p * Ne + c)] = br * ir - bi * ii;
-                            Sb[2 * (p * Ne + c) + 1] = br * ii + bi * ir;
-                        }
-                        __syncthreads();
-                        for (int idx = tid; idx < Ne * Ne; idx += B) {
-                            const int r = idx / Ne, c = idx - r * Ne;
-                            if (r == p) continue;
-                            const double fr = pcol[2 * r], fi = pcol[2 * r + 1];
-                            const double xr = (c == p) ? 0.0 : Sb[2 * idx], xi = (c == p) ? 0.0 : Sb[2 * idx + 1];
-                            const double yr = Sb[2 * (p * Ne + c)], yi = Sb[2 * (p * Ne + c) + 1];
-                            Sb[2 * idx] = xr - (fr * yr - fi * yi);
-                            Sb[2 * idx + 1] = xi - (fr * yi + fi * yr);
-                        }
-                    }
-                    __syncthreads();
-                    if (!gj_singular) {  // undo the row interchanges as column interchanges: Sb = S^-1
-                        for (int p = Ne - 1; p >= 0; --p) {
-                            const int q = piv[p];
-                            if (q != p) {
-                                for (int r = tid; r < Ne; r += B) {
-                                    const double ar = Sb[2 * (r * Ne + p)], ai = Sb[2 * (r * Ne + p) + 1];
-                                    Sb[2 * (r * Ne + p)] = Sb[2 * (r * Ne + q)];
-                                    Sb[2 * (r * Ne + p) + 1] = Sb[2 * (r * Ne + q) + 1];
-                                    Sb[2 * (r * Ne + q)] = ar;
-                                    Sb[2 * (r * Ne + q) + 1] = ai;
-                                }
-                            }
-                            __syncthreads();
-                        }
-                    }
+                    __syncthreads();  // S^-1 and the unoccupied states are in place
                     // P(n -> m) = 2 dt Re((psi_m S^-1)_n) v_dot_d[m, n]: det(S with row n replaced by
                     // psi_m) = det(S) (psi_m S^-1)_n, so Re(det S conj(det S_{n<-m})) / |det S|^2 is that real part.
                     // pass 1: per-electron totals, partial sums over interleaved chunks of unoccupied states
@@ -920,7 +850,7 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(NT <= 4
                         const int n = tid % Ne, ch = tid / Ne;
                         const int o = occ[n];
                         double part_sum = 0.0;
-                        for (int mi = gj_singular ? Nu : ch; mi < Nu; mi += nch) {  // no hop from a singular S
+                        for (int mi = ch; mi < Nu; mi += nch) {
                             const int m = unocc[mi];
                             double zr = 0.0;
                             for (int e = 0; e < Ne; ++e)
@@ -937,15 +867,19 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(NT <= 4
                         pcol[n] = sn;
                     }
                     __syncthreads();
-                    if (tid == 0) {  // the electron whose cumulative total passes the uniform, if any
+                    if (w == 0) {  // the electron whose cumulative total passes the uniform, if any
+                        const double mine = l < Ne ? pcol[l] : 0.0;
                         double cum = 0.0;
                         int hn = -1;
                         for (int n = 0; n < Ne; ++n) {
-                            if (rnd < cum + pcol[n]) { hn = n; break; }
-                            cum += pcol[n];
+                            const double pn = readlane_f64(mine, n);
+                            if (rnd < cum + pn) { hn = n; break; }
+                            cum += pn;
                         }
-                        scal[3] = (double)hn;
-                        scal[4] = cum;
+                        if (l == 0) {
+                            scal[3] = (double)hn;
+                            scal[4] = cum;
+                        }
                     }
                     __syncthreads();
                     const int hsel = (int)scal[3];
@@ -1062,21 +996,25 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(NT <= 4
     }
 }
 
-// Determinants of nmat complex Ne x Ne matrices (re, im planes, row-major) by wave_det, one
-// wavefront per matrix: the test hook of the IESH estimate's determinant.
-__global__ __launch_bounds__(64) void wave_det_kernel(const double* __restrict__ re, const double* __restrict__ im,
-                                                      int Ne, double* __restrict__ out) {
-    extern __shared__ double S[];  // 2 Ne LD
-    const int LD = Ne | 1;
+// Determinants of nmat complex Ne x Ne matrices (re, im planes, row-major) by block_inverse, one
+// workgroup per matrix: the test hook of the IESH estimate's determinant.
+__global__ __launch_bounds__(256) void det_kernel(const double* __restrict__ re, const double* __restrict__ im, int Ne,
+                                                  double* __restrict__ out) {
+    __shared__ double buf[2 * 136];
+    __shared__ int piv[kIeMaxNe];
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
     const size_t base = (size_t)blockIdx.x * Ne * Ne;
-    for (int idx = threadIdx.x; idx < Ne * Ne; idx += 64) {
-        const int j = idx / Ne, e = idx - j * Ne;
-        S[j * LD + e] = re[base + idx];
-        S[Ne * LD + j * LD + e] = im[base + idx];
+    double xr[16], xi[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+        const int c = w + 4 * j;
+        const bool in = l < Ne && c < Ne;
+        xr[j] = in ? re[base + (size_t)l * Ne + c] : 0.0;
+        xi[j] = in ? im[base + (size_t)l * Ne + c] : 0.0;
     }
-    __syncthreads();
     double dr, di;
-    const bool ok = wave_det(S, S + Ne * LD, LD, Ne, dr, di);
+    int myp, rot;
+    const bool ok = block_inverse<4, 16>(xr, xi, Ne, w, l, buf, piv, dr, di, myp, rot);
     if (threadIdx.x == 0) {
         out[3 * blockIdx.x] = dr;
         out[3 * blockIdx.x + 1] = di;
@@ -1091,7 +1029,7 @@ __global__ __launch_bounds__(64) void wave_det_kernel(const double* __restrict__
 // wavefront per trajectory, root ir on lane ir % 64.
 __global__ __launch_bounds__(256) void ie_initial_energies(const IeshArgs A, int diabatic, double* __restrict__ W) {
     __shared__ double eps[kIeMaxStates];
-    for (int k = threadIdx.x; k < A.M; k += blockDim.x) eps[k] = A.a + k * A.de;
+    for (int k = threadIdx.x; k < kIeMaxStates; k += blockDim.x) eps[k] = k < A.M ? A.a + k * A.de : kFarPole;
     __syncthreads();
     const int64_t traj = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     if (traj >= A.ntraj) return;
@@ -1236,12 +1174,12 @@ __global__ __launch_bounds__(256) void ie_diabatic_orbitals(int64_t ntraj, int N
     for (uint64_t w = tk_hi; w; w &= w - 1) occ0[traj * Ne + e++] = 64 + __ffsll((unsigned long long)w) - 1;
 }
 
-// S as two planes with an odd row stride (determinant), or interleaved Ne x Ne (inverse)
-int ie_sb_len(int N, int Ne) { (void)N; return 2 * Ne * (Ne | 1); }
+// S^-1, interleaved complex
+int ie_sb_len(int Ne) { return 2 * Ne * Ne; }
 
 size_t ie_lds_bytes(int NT, int cw, int N, int Ne, int P) {
     const int NP = 16 * NT;
-    return sizeof(double) * ((size_t)NP * cw + ie_sb_len(N, Ne) + 3 * NP + 8 + std::max(NP, 2 * kIeMaxNe) + 8 * kIeMaxNe + 8) +
+    return sizeof(double) * ((size_t)NP * cw + ie_sb_len(Ne) + 3 * NP + 8 + std::max(NP, 2 * kIeMaxNe) + 8 * kIeMaxNe + 8) +
            sizeof(int) * (2 * kIeMaxNe + 2 * NP) + (P > 1 ? sizeof(double) * (5 * 64 + 2 * (size_t)NP) : 0);
 }
 
@@ -1500,7 +1438,7 @@ int32_t ie_run(nqcd_handle_t* h, double t0, int64_t nsteps, const nqcd_term_desc
     A.ntraj = n;
     A.nsteps = nsteps;
     A.N = N; A.M = md.M; A.Ne = Ne; A.cw = 16 * CT;
-    A.sb_len = ie_sb_len(N, Ne);
+    A.sb_len = ie_sb_len(Ne);
     A.method = (h->prob.method == NQCD_METHOD_IESH) ? 0 : 1;
     A.rescaling = h->prob.rescaling;
     A.estimate = h->prob.disable_estimate ? 0 : 1;
@@ -1581,10 +1519,8 @@ int32_t ie_test_det(nqcd_handle_t* h, const double* re, const double* im, int32_
     HIPCHK(h, o.ensure(sizeof(double) * 3 * nmat));
     hipError_t e = hipMemcpy(a.p, re, sizeof(double) * n, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(b.p, im, sizeof(double) * n, hipMemcpyHostToDevice);
-    const size_t lds = sizeof(double) * 2 * Ne * (Ne | 1);
-    if (e == hipSuccess) e = hipFuncSetAttribute((const void*)wave_det_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(wave_det_kernel, dim3(nmat), dim3(64), lds, h->stream, a.as<double>(), b.as<double>(), Ne, o.as<double>());
+        hipLaunchKernelGGL(det_kernel, dim3(nmat), dim3(256), 0, h->stream, a.as<double>(), b.as<double>(), Ne, o.as<double>());
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpy(out, o.p, sizeof(double) * 3 * nmat, hipMemcpyDeviceToHost);
