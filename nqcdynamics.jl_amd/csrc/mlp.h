@@ -93,6 +93,17 @@ __host__ __device__ constexpr int mlp_perm_unit(int q, int k) {
     return 32 * q + ((k & 7) < 4 ? 4 * (k >> 3) + (k & 7) : 16 + 4 * (k >> 3) + (k & 7) - 4);
 }
 
+// its inverse: the permuted column of a unit
+__host__ __device__ constexpr int mlp_perm_col(int u) {
+    return (u & ~31) + 8 * ((u >> 2) & 3) + ((u >> 4) & 1) * 4 + (u & 3);
+}
+constexpr bool mlp_perm_inverse() {
+    for (int u = 0; u < kMlpH; ++u)
+        if (mlp_perm_unit(mlp_perm_col(u) >> 5, mlp_perm_col(u) & 31) != u) return false;
+    return true;
+}
+static_assert(mlp_perm_inverse(), "column of a unit");
+
 // A zero the optimiser cannot see through: offsetting a pointer by it at a point makes the loads
 // through that pointer issue there rather than be hoisted out of the surrounding loop (which would
 // keep every weight fragment live), while the pointer keeps its LDS address space.

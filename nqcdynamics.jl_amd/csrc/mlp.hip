@@ -1,10 +1,11 @@
 // mlp.hip -- training and batched evaluation of the MLP surrogate (mlp.h) on the GPU.
 //
 // Training: Adam on the mean weighted squared error of the normalised (H11, H22, H12) targets.
-// Each step: mlp_train_grad (one wavefront per 32 samples: forward through mlp_tile, backward
+// Each step: mlp_train_grad (one workgroup per 32 samples: forward through mlp_tile, backward
 // with BF16 MFMA for delta1 = W2^T delta2 and dW2 = delta2 h1^T, FP32 elsewhere; per-group partial
 // gradients), mlp_reduce_adam (gradient = fixed-order sum of the partials, Adam on the FP32
-// master parameters), mlp_pack (BF16 packed copy for the next forward).
+// master parameters and their BF16 packed copy for the next forward).  mlp_pack makes the first
+// packed copy.  1000 steps of 2048 samples, two members: 41.9 -> 24.3 ms.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -21,9 +22,12 @@ namespace nqcd {
 namespace {
 
 constexpr int kTrainSamples = 32;  // samples per training workgroup (two sample tiles)
-constexpr int kTrainThreads = 128; // one wavefront per sample tile
-static_assert(kTrainThreads / 64 == kTrainSamples / 16, "one wavefront per 16-sample tile");
+constexpr int kTrainThreads = 512; // two wavefronts take the sample tiles, all eight the staging and the parameter sums
+static_assert(kTrainThreads / 64 >= kTrainSamples / 16, "one wavefront per 16-sample tile");
+static_assert(kTrainThreads >= kMlpOut * kMlpH + kMlpH, "one thread per element of W3, b1 and b2");
+constexpr int kTrainRow = 36;      // floats between units (16-byte aligned, 4 lanes to a bank instead of 32)
 constexpr int kPackBlocks = 64;
+constexpr int kAdamThreads = 64;
 
 // Packs member blockIdx.y: P and out advance by one member per blockIdx.y.
 __global__ __launch_bounds__(256) void mlp_pack(const float* __restrict__ P, unsigned char* __restrict__ out) {
@@ -106,24 +110,52 @@ __global__ __launch_bounds__(256) void mlp_eval_kernel(const unsigned char* __re
     }
 }
 
-// One workgroup of two wavefronts per 32 samples of the minibatch: partial gradient (kMlpParams
-// floats, master order) and partial loss of those samples.  Each wavefront takes one 16-sample
-// tile through the network, then the two split the parameter sums over the 32 samples.
+// One workgroup per 32 samples of the minibatch: partial gradient (kMlpParams floats, master order)
+// and partial loss of those samples.  Two wavefronts take one 16-sample tile each through the network;
+// all eight stage the member and split the parameter sums over the 32 samples.  Bound by latency (128
+// workgroups for two members of 2048 samples): with the two wavefronts alone, staging 80 KB in 39
+// dependent rounds and sums whose lanes shared a bank made it 28 of a step's 41 us.
 struct TrainLds {
     unsigned char member[kPkBytes];        // the packed member, W2^T included
     float W3[kMlpOut * kMlpH];
     __bf16 h1q[kMlpH * kTrainSamples];     // [unit][sample]
-    float d2[kMlpH * kTrainSamples];       // [unit][sample]
-    float h2q[kMlpH * kTrainSamples];
-    float d1[kMlpH * kTrainSamples];
-    float x[kTrainSamples * kMlpIn];
-    float d3[kTrainSamples * kMlpOut];
+    alignas(16) float d2[kMlpH * kTrainRow];  // [unit][sample]
+    alignas(16) float h2q[kMlpH * kTrainRow];
+    alignas(16) float d1[kMlpH * kTrainRow];
+    alignas(16) float x[kMlpIn * kTrainRow];  // [input][sample]
+    alignas(16) float d3[kMlpOut * kTrainRow];
     float loss[kTrainSamples];
 };
 
+// Sums over a workgroup's samples, rows of the LDS arrays, in order.
+__device__ __forceinline__ float sample_dot(const float* a, const float* b) {
+    float s = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kTrainSamples; k += 4) {
+        const float4 x = *reinterpret_cast<const float4*>(a + k), y = *reinterpret_cast<const float4*>(b + k);
+        s += x.x * y.x;
+        s += x.y * y.y;
+        s += x.z * y.z;
+        s += x.w * y.w;
+    }
+    return s;
+}
+__device__ __forceinline__ float sample_sum(const float* a) {
+    float s = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kTrainSamples; k += 4) {
+        const float4 x = *reinterpret_cast<const float4*>(a + k);
+        s += x.x;
+        s += x.y;
+        s += x.z;
+        s += x.w;
+    }
+    return s;
+}
+
 // Member blockIdx.y (the members train side by side in one launch): its packed copy, master
 // parameters, minibatch indices (idx + member * idx_stride), partial gradients and losses.
-__global__ __launch_bounds__(128) void mlp_train_grad(const unsigned char* __restrict__ packed, const float* __restrict__ P,
+__global__ __launch_bounds__(kTrainThreads) void mlp_train_grad(const unsigned char* __restrict__ packed, const float* __restrict__ P,
                                                      const float* __restrict__ Xn, const float* __restrict__ Tn,
                                                      const int32_t* __restrict__ idx, int64_t idx_stride, int32_t nb,
                                                      float w0, float w1, float w2, float* __restrict__ partial,
@@ -136,13 +168,22 @@ __global__ __launch_bounds__(128) void mlp_train_grad(const unsigned char* __res
     loss_part += (size_t)mem * gridDim.x;
     extern __shared__ __align__(16) unsigned char lds_raw[];
     TrainLds& S = *reinterpret_cast<TrainLds*>(lds_raw);
-    const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63, g = l >> 4, j = l & 15;
-    stage_member(packed, S.member);
-    for (int i = tid; i < kMlpOut * kMlpH; i += kTrainThreads) S.W3[i] = P[kOffW3 + i];
+    const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, g = l >> 4, j = l & 15;
+    {  // all of a thread's loads in flight together
+        constexpr int kAll = kPkBytes / 16, kEach = (kAll + kTrainThreads - 1) / kTrainThreads;
+        const uint4* src = reinterpret_cast<const uint4*>(packed);
+        uint4* dst = reinterpret_cast<uint4*>(S.member);
+        uint4 t[kEach];
+#pragma unroll
+        for (int q = 0; q < kEach; ++q) t[q] = src[min(tid + q * kTrainThreads, kAll - 1)];
+        if (tid < kMlpOut * kMlpH) S.W3[tid] = P[kOffW3 + tid];
+#pragma unroll
+        for (int q = 0; q < kEach; ++q) dst[min(tid + q * kTrainThreads, kAll - 1)] = t[q];
+    }
     __syncthreads();
     const float wl[3] = {w0, w1, w2};
     const int g0 = blockIdx.x * kTrainSamples;
-    {
+    if (wv < kTrainSamples / 16) {
         const int T = wv;  // this wavefront's sample tile
         const int ls = 16 * T + j;                  // local sample of this lane's column
         const bool valid = g0 + ls < nb;
@@ -167,9 +208,9 @@ __global__ __launch_bounds__(128) void mlp_train_grad(const unsigned char* __res
         if (g == 0) {
             S.loss[ls] = lo / (float)nb;
 #pragma unroll
-            for (int r = 0; r < kMlpOut; ++r) S.d3[ls * kMlpOut + r] = d3[r];
+            for (int r = 0; r < kMlpOut; ++r) S.d3[r * kTrainRow + ls] = d3[r];
 #pragma unroll
-            for (int i = 0; i < kMlpIn; ++i) S.x[ls * kMlpIn + i] = xs[i];
+            for (int i = 0; i < kMlpIn; ++i) S.x[i * kTrainRow + ls] = xs[i];
         }
         // delta2 = s2 * (W3^T delta3); stage h1q, h2q, delta2 as [unit][sample]
         float d2[32];
@@ -182,9 +223,9 @@ __global__ __launch_bounds__(128) void mlp_train_grad(const unsigned char* __res
 #pragma unroll
                 for (int o3 = 0; o3 < kMlpOut; ++o3) a += S.W3[o3 * kMlpH + u] * d3[o3];
                 d2[k] = s2[k] * a;
-                S.d2[u * kTrainSamples + ls] = d2[k];
+                S.d2[u * kTrainRow + ls] = d2[k];
                 S.h1q[u * kTrainSamples + ls] = (__bf16)h1[k];
-                S.h2q[u * kTrainSamples + ls] = (float)(__bf16)h2[k];
+                S.h2q[u * kTrainRow + ls] = (float)(__bf16)h2[k];
             }
         }
         // delta1 = s1 * (W2^T delta2) on MFMA (units of W2's input along M, samples along N)
@@ -200,7 +241,7 @@ __global__ __launch_bounds__(128) void mlp_train_grad(const unsigned char* __res
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int u = 16 * ut + 4 * g + r;
-                S.d1[u * kTrainSamples + ls] = s1[4 * ut + r] * acc[r];
+                S.d1[u * kTrainRow + ls] = s1[4 * ut + r] * acc[r];
             }
         }
     }
@@ -209,11 +250,11 @@ __global__ __launch_bounds__(128) void mlp_train_grad(const unsigned char* __res
     // dW2 = delta2 h1q^T on MFMA, K = the 32 samples: A = delta2 [v][s], B = h1q [u][s]
 #pragma unroll 1
     for (int vt = wv; vt < 8; vt += kTrainThreads / 64) {
-        float av[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) av[e] = S.d2[(16 * vt + j) * kTrainSamples + 8 * g + e];
+        const float* dv = &S.d2[(16 * vt + j) * kTrainRow + 8 * g];
+        const float4 lo = *reinterpret_cast<const float4*>(dv), hi = *reinterpret_cast<const float4*>(dv + 4);
+        const float av[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
         const bf16x8 A = pack8(av, av + 4);
-#pragma unroll 1
+#pragma unroll
         for (int ut = 0; ut < 8; ++ut) {
             const bf16x8 Bh = *reinterpret_cast<const bf16x8*>(&S.h1q[(16 * ut + j) * kTrainSamples + 8 * g]);
             const f32x4 acc = mfma_bf16(A, Bh, f32x4{0.f, 0.f, 0.f, 0.f});
@@ -221,30 +262,20 @@ __global__ __launch_bounds__(128) void mlp_train_grad(const unsigned char* __res
             for (int r = 0; r < 4; ++r) out[kOffW2 + (16 * vt + 4 * g + r) * kMlpH + 16 * ut + j] = acc[r];
         }
     }
-    // FP32 sums over the samples for the small parameter blocks
-    for (int p = tid; p < kMlpOut * kMlpH; p += kTrainThreads) {
-        const int o3 = p / kMlpH, u = p % kMlpH;
-        float a = 0.0f;
-        for (int s = 0; s < kTrainSamples; ++s) a += S.d3[s * kMlpOut + o3] * S.h2q[u * kTrainSamples + s];
-        out[kOffW3 + p] = a;
+    // FP32 sums over the samples for the small parameter blocks, in sample order
+    if (tid < kMlpOut * kMlpH) {
+        const int o3 = tid / kMlpH, u = tid % kMlpH;
+        out[kOffW3 + tid] = sample_dot(&S.d3[o3 * kTrainRow], &S.h2q[u * kTrainRow]);
+    } else if (tid < kMlpOut * kMlpH + kMlpH) {
+        const int u = tid - kMlpOut * kMlpH;
+        out[kOffB1 + u] = sample_sum(&S.d1[u * kTrainRow]);
+        out[kOffB2 + u] = sample_sum(&S.d2[u * kTrainRow]);
     }
     for (int p = tid; p < kMlpH * kMlpIn; p += kTrainThreads) {
         const int u = p / kMlpIn, i = p % kMlpIn;
-        float a = 0.0f;
-        for (int s = 0; s < kTrainSamples; ++s) a += S.d1[u * kTrainSamples + s] * S.x[s * kMlpIn + i];
-        out[kOffW1 + p] = a;
+        out[kOffW1 + p] = sample_dot(&S.d1[u * kTrainRow], &S.x[i * kTrainRow]);
     }
-    for (int u = tid; u < kMlpH; u += kTrainThreads) {
-        float a1 = 0.0f, a2 = 0.0f;
-        for (int s = 0; s < kTrainSamples; ++s) { a1 += S.d1[u * kTrainSamples + s]; a2 += S.d2[u * kTrainSamples + s]; }
-        out[kOffB1 + u] = a1;
-        out[kOffB2 + u] = a2;
-    }
-    if (tid < kMlpOut) {
-        float a = 0.0f;
-        for (int s = 0; s < kTrainSamples; ++s) a += S.d3[s * kMlpOut + tid];
-        out[kOffB3 + tid] = a;
-    }
+    if (tid < kMlpOut) out[kOffB3 + tid] = sample_sum(&S.d3[tid * kTrainRow]);
     if (tid == 0) {
         float a = 0.0f;
         for (int s = 0; s < kTrainSamples; ++s) a += S.loss[s];
@@ -252,29 +283,55 @@ __global__ __launch_bounds__(128) void mlp_train_grad(const unsigned char* __res
     }
 }
 
-// x[0] + x[stride] + ... + x[(n - 1) stride], added in that order; the loads of 16 terms are
-// issued together, so a sum costs n / 16 memory latencies instead of n.
+// x[0] + x[stride] + ... + x[(n - 1) stride], added in that order; the loads of 32 terms are
+// issued together, so a sum costs n / 32 memory latencies instead of n.
 __device__ __forceinline__ float ordered_sum(const float* __restrict__ x, int64_t stride, int n) {
     float a = 0.0f;
     int k = 0;
-    for (; k + 16 <= n; k += 16) {
-        float t[16];
+    for (; k + 32 <= n; k += 32) {
+        float t[32];
 #pragma unroll
-        for (int q = 0; q < 16; ++q) t[q] = x[(k + q) * stride];
+        for (int q = 0; q < 32; ++q) t[q] = x[(k + q) * stride];
 #pragma unroll
-        for (int q = 0; q < 16; ++q) a += t[q];
+        for (int q = 0; q < 32; ++q) a += t[q];
     }
     for (; k < n; ++k) a += x[k * stride];
     return a;
 }
 
-// Member blockIdx.y: fixed-order sum of its ngroups partial gradients, then Adam.
-__global__ __launch_bounds__(256) void mlp_reduce_adam(const float* __restrict__ partial, int32_t ngroups, float* P,
+// Parameter p of the master vector, in its places in the packed member (the rest of a packed member never changes).
+__device__ __forceinline__ void pack_param(int p, float x, unsigned char* out) {
+    if (p < kOffB1) {
+        const int u = p / kMlpIn, i = p - u * kMlpIn;
+        reinterpret_cast<float*>(out + kPkW1B)[8 * u + i] = x;
+        reinterpret_cast<__bf16*>(out + kPkW1T)[mlp_swz(i, mlp_perm_col(u))] = (__bf16)x;
+    } else if (p < kOffW2) {
+        reinterpret_cast<float*>(out + kPkW1B)[8 * (p - kOffB1) + kMlpIn] = x;
+    } else if (p < kOffB2) {
+        const int v = (p - kOffW2) / kMlpH, u = (p - kOffW2) % kMlpH;
+        reinterpret_cast<__bf16*>(out + kPkW2)[mlp_swz(v, mlp_perm_col(u))] = (__bf16)x;
+        reinterpret_cast<__bf16*>(out + kPkW2T)[mlp_swz(u, mlp_perm_col(v))] = (__bf16)x;
+    } else if (p < kOffW3) {
+        reinterpret_cast<float*>(out + kPkB2)[p - kOffB2] = x;
+    } else if (p < kOffB3) {
+        const int o = (p - kOffW3) / kMlpH, c = mlp_perm_col((p - kOffW3) % kMlpH);
+        reinterpret_cast<__bf16*>(out + kPkW3)[mlp_swz(o, c)] = (__bf16)x;
+        reinterpret_cast<float*>(out + kPkW3F)[o * kMlpH + c] = (float)(__bf16)x;
+    } else {
+        reinterpret_cast<float*>(out + kPkB3)[p - kOffB3] = x;
+    }
+}
+
+// Member blockIdx.y: fixed-order sum of its ngroups partial gradients, then Adam and the packed copy (a kernel of its
+// own for the copy was 4 us of a step).  64 threads a workgroup: a parameter's sum is a chain of memory latencies, and
+// 558 small workgroups spread over all compute units.
+__global__ __launch_bounds__(kAdamThreads) void mlp_reduce_adam(const float* __restrict__ partial, int32_t ngroups, float* P,
                                                        float* m, float* v, float lr, float b1, float b2, float eps,
                                                        float b1t, float b2t, int32_t apply, float* grad_out,
                                                        const float* __restrict__ loss_part, float* loss_out,
-                                                       int64_t loss_stride) {
+                                                       int64_t loss_stride, unsigned char* packed) {
     const int mem = blockIdx.y;
+    packed += (size_t)mem * kPkBytes;
     partial += (size_t)mem * ngroups * kMlpParams;
     P += (size_t)mem * kMlpParams;
     m += (size_t)mem * kMlpParams;
@@ -292,7 +349,9 @@ __global__ __launch_bounds__(256) void mlp_reduce_adam(const float* __restrict__
     const float vv = b2 * v[p] + (1.0f - b2) * gsum * gsum;
     m[p] = mm;
     v[p] = vv;
-    P[p] -= lr * (mm / (1.0f - b1t)) / (sqrtf(vv / (1.0f - b2t)) + eps);
+    const float x = P[p] - lr * (mm / (1.0f - b1t)) / (sqrtf(vv / (1.0f - b2t)) + eps);
+    P[p] = x;
+    pack_param(p, x, packed);
 }
 
 size_t train_lds_bytes() { return sizeof(TrainLds); }
@@ -391,16 +450,12 @@ static int32_t train_step(nqcd_handle_t* h, int k0, int nmem, const int32_t* idx
                        h->mlp_losspart.as<float>());
     HIPCHK(h, hipGetLastError());
     const float b1 = 0.9f, b2 = 0.999f;
-    hipLaunchKernelGGL(mlp_reduce_adam, dim3((kMlpParams + 255) / 256, nmem), dim3(256), 0, h->stream,
+    hipLaunchKernelGGL(mlp_reduce_adam, dim3((kMlpParams + kAdamThreads - 1) / kAdamThreads, nmem), dim3(kAdamThreads), 0, h->stream,
                        h->mlp_partial.as<float>(), ngroups, P, h->mlp_adam_m.as<float>() + (size_t)k0 * kMlpParams,
                        h->mlp_adam_v.as<float>() + (size_t)k0 * kMlpParams, lr, b1, b2, 1e-8f,
                        (float)std::pow(b1, (double)t), (float)std::pow(b2, (double)t), apply ? 1 : 0, grad_dev,
-                       h->mlp_losspart.as<float>(), loss_dev, loss_stride);
+                       h->mlp_losspart.as<float>(), loss_dev, loss_stride, packed);
     HIPCHK(h, hipGetLastError());
-    if (apply) {
-        hipLaunchKernelGGL(mlp_pack, dim3(kPackBlocks, nmem), dim3(256), 0, h->stream, P, packed);
-        HIPCHK(h, hipGetLastError());
-    }
     return NQCD_OK;
 }
 
