@@ -78,12 +78,12 @@ __device__ __forceinline__ Fssh2Hot<D> fssh2_hot(const Fssh2Args& A) {
 }
 
 template <int D, typename R>
-__device__ __forceinline__ void eval_cache(Lane2<D, R>& L, bool track, double& E0, double& E1, double G00[D],
-                                           double G11[D], double G01[D]) {
+__device__ __forceinline__ void eval_cache(Lane2<D, R>& L, bool track, double& E0, double& E1, double& inv_gap,
+                                           double G00[D], double G11[D], double G01[D]) {
     static_assert(D == 1, "one-dimensional models");
     R v11, v22, v12, d11, d22, d12;
     model1d_eval_lane<R>(L.m, L.r[0], v11, v22, v12, d11, d22, d12);
-    eigen2((double)v11, (double)v12, (double)v22, E0, E1, L.U, track);
+    eigen2_gap((double)v11, (double)v12, (double)v22, E0, E1, inv_gap, L.U, track);
     rotate_derivative(L.U, (double)d11, (double)d22, (double)d12, G00[0], G11[0], G01[0]);
 }
 
@@ -157,8 +157,8 @@ __device__ __forceinline__ void load_traj(const Fssh2Args* Ap, const Fssh2Hot<D>
         st = (u < a) ? 0 : 1;
     }
     L.st = st;
-    double E0, E1, G00[D], G11[D], G01[D];
-    eval_cache(L, false, E0, E1, G00, G11, G01);  // initialize! (bab_electronics.jl:48-59)
+    double E0, E1, inv_gap, G00[D], G11[D], G01[D];
+    eval_cache(L, false, E0, E1, inv_gap, G00, G11, G01);  // initialize! (bab_electronics.jl:48-59)
     set_accel(H, L, G00, G11, G01);
     L.dEc = 0.0; L.wc = 0.0; L.tc = 0.0;  // zero buffers stamped t = 0 (electronic_dynamics.jl:118-127)
     L.t = A.t0;
@@ -246,20 +246,19 @@ __device__ __forceinline__ void step_traj(const Fssh2Args* Ap, const Fssh2Args& 
     for (int I = 0; I < D; ++I) vt[I] = L.v[I] + hdt * L.k[I];           // step_B!
 #pragma unroll
     for (int I = 0; I < D; ++I) L.r[I] = L.r[I] + dtR * vt[I];           // step_A!
-    double E0, E1, G00[D], G11[D], G01[D];
-    eval_cache(L, true, E0, E1, G00, G11, G01);                          // update_cache!
+    double E0, E1, inv_gap, G00[D], G11[D], G01[D];
+    eval_cache(L, true, E0, E1, inv_gap, G00, G11, G01);                          // update_cache!
     set_accel(H, L, G00, G11, G01);                                      // sigma of the step start
 #pragma unroll
     for (int I = 0; I < D; ++I) L.v[I] = vt[I] + hdt * L.k[I];           // step_B!
     const double gap = E1 - E0;
-    const double inv_gap = 1.0 / gap;
     double d01[D];
     double w = 0.0;
 #pragma unroll
     for (int I = 0; I < D; ++I) { d01[I] = G01[I] * inv_gap; w += d01[I] * (double)L.v[I]; }
     const double tn = L.t + H.dt;
     const double dEn = E0 - E1;
-    const double inv = 1.0 / (tn - L.tc);
+    const double inv = nr_rcp(tn - L.tc);
     Interp2 P;
     P.dE0 = L.dEc; P.dE1 = (dEn - L.dEc) * inv; P.w0 = L.wc; P.w1 = (w - L.wc) * inv;
     propagate2<R>(P, L.s, L.t, L.tc, H.dt, H.nsub);

@@ -114,8 +114,10 @@ __device__ __forceinline__ void map_electronic_step(const LaneN<NM, double>& L, 
     double vd[NM], vo[NP > 0 ? NP : 1], dd[NM], dof[NP > 0 ? NP : 1];
     ns_model<NM, double>(L, x, vd, vo, dd, dof);
     double w[NM];
-    if constexpr (NM == 2) eigen2(vd[0], vo[0], vd[1], w[0], w[1], Z, false);
-    else ns_eigen<NM>(NM, vd, vo, w, Z, false, true);
+    if constexpr (NM == 2) {
+        double inv_gap;
+        eigen2_gap(vd[0], vo[0], vd[1], w[0], w[1], inv_gap, Z, false);
+    } else ns_eigen<NM>(NM, vd, vo, w, Z, false, true);
     double vbar = 0.0, dbar = 0.0;
     tr = 0.0;
 #pragma unroll

@@ -365,6 +365,35 @@ __device__ __forceinline__ void eigen2(double a, double c, double d, double& E0,
     U[0] = u00; U[1] = u01; U[2] = u10; U[3] = u11;
 }
 
+// The same with 1 / (E1 - E0), for the steps of the two-state kernels: one reciprocal square root serves the radius,
+// its inverse and, with the eigenvector's norm^2 = 2 rad (rad + |h|), a second one the vector (within an ulp), in place
+// of two square roots and two divisions.  Radii whose square could leave the range of a double take those.
+__device__ __forceinline__ void eigen2_gap(double a, double c, double d, double& E0, double& E1, double& inv_gap, double U[4],
+                                           bool track) {
+    const double mean = 0.5 * (a + d), h = 0.5 * (a - d);
+    const double x = fma(h, h, c * c);
+    if (!(x > 1e-280 && x < 1e280)) {
+        eigen2(a, c, d, E0, E1, U, track);
+        inv_gap = 1.0 / (E1 - E0);
+        return;
+    }
+    const double y = nr_rsq(x);
+    double rad = x * y;
+    rad = fma(fma(-rad, rad, x), 0.5 * y, rad);
+    E0 = mean - rad;
+    E1 = mean + rad;
+    inv_gap = 0.5 * y;
+    const double far = rad + fabs(h), n = nr_rsq(2.0 * rad * far);
+    const double big = far * n, small = c * n;
+    const double p = h >= 0.0 ? big : small, q = h >= 0.0 ? small : big;  // eigenvector of E1
+    const bool f0 = track ? p * U[2] < q * U[0] : (fabs(p) > fabs(q) ? p : -q) < 0.0;
+    const bool f1 = track ? p * U[1] + q * U[3] < 0.0 : (fabs(q) > fabs(p) ? q : p) < 0.0;
+    U[0] = f0 ? q : -q;
+    U[2] = f0 ? -p : p;
+    U[1] = f1 ? -p : p;
+    U[3] = f1 ? -q : q;
+}
+
 // G = U^T dV U for dV = [[d11, d12],[d12, d22]]; returns G00, G11, G01.
 __device__ __forceinline__ void rotate_derivative(const double U[4], double d11, double d22, double d12,
                                                   double& G00, double& G11, double& G01) {

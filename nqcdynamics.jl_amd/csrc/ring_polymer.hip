@@ -121,8 +121,8 @@ __device__ __forceinline__ double bead_force(const RpArgs& A, const ModelRegs& m
     if (!E || A.method != 2) return (double)surface_gradient<R>(m, x, E && A.method == 1, st);
     R v11, v22, v12, d11, d22, d12;
     model1d_eval<R>(m, x, v11, v22, v12, d11, d22, d12);
-    double E0, E1, G00, G11, G01;
-    eigen2((double)v11, (double)v12, (double)v22, E0, E1, Ub, track);
+    double E0, E1, inv_gap, G00, G11, G01;
+    eigen2_gap((double)v11, (double)v12, (double)v22, E0, E1, inv_gap, Ub, track);
     rotate_derivative(Ub, (double)d11, (double)d22, (double)d12, G00, G11, G01);
     return G00 * a + G11 * b + 2.0 * G01 * sx;
 }
@@ -173,14 +173,14 @@ __device__ __forceinline__ void rp_elec_propagate(const AT& A, const ModelRegs& 
                                                   double tn, RpElec& E) {
     R v11, v22, v12, d11, d22, d12;
     model1d_eval<R>(m, rc, v11, v22, v12, d11, d22, d12);
-    double E0c, E1c, G00c, G11c, G01c;
-    eigen2((double)v11, (double)v12, (double)v22, E0c, E1c, E.Uc, true);
+    double E0c, E1c, inv_gap, G00c, G11c, G01c;
+    eigen2_gap((double)v11, (double)v12, (double)v22, E0c, E1c, inv_gap, E.Uc, true);
     rotate_derivative(E.Uc, (double)d11, (double)d22, (double)d12, G00c, G11c, G01c);
     E.gap = E1c - E0c;
-    E.d01 = G01c / E.gap;
+    E.d01 = G01c * inv_gap;
     const double w = E.d01 * vc;
     const double dEn = E0c - E1c;
-    const double inv = 1.0 / (tn - E.tc);
+    const double inv = nr_rcp(tn - E.tc);
     Interp2 Pi;
     Pi.dE0 = E.dEc; Pi.dE1 = (dEn - E.dEc) * inv; Pi.w0 = E.wc; Pi.w1 = (w - E.wc) * inv;
     propagate2<R>(Pi, E.s, t, E.tc, A.dt, A.nsub);

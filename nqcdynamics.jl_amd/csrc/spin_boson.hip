@@ -231,7 +231,8 @@ __device__ __forceinline__ void sb_body(const SbArgs* __restrict__ Ap, SbVec<R>*
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        eigen2(eps + (double)Xn, Delta, -eps - (double)Xn, E0, E1, U, true);  // update_cache!
+        double inv_gap;
+        eigen2_gap(eps + (double)Xn, Delta, -eps - (double)Xn, E0, E1, inv_gap, U, true);  // update_cache!
         rotate_sz(U, g00, g11, g01);
         {
             const double aa = 0.5 * (tr + s.q), bb = 0.5 * (tr - s.q);
@@ -271,11 +272,11 @@ __device__ __forceinline__ void sb_body(const SbArgs* __restrict__ Ap, SbVec<R>*
             }
         }
         const double gap = E1 - E0;
-        const double d01c = g01 / gap;               // d_j[0][1] = c_j * d01c
+        const double d01c = g01 * inv_gap;             // d_j[0][1] = c_j * d01c
         const double w = d01c * (double)Vc;
         const double tn = t + dt;
         const double dEn = E0 - E1;
-        const double inv = 1.0 / (tn - tc);
+        const double inv = nr_rcp(tn - tc);
         Interp2 P;
         P.dE0 = dEc; P.dE1 = (dEn - dEc) * inv; P.w0 = wc; P.w1 = (w - wc) * inv;
         // 100 modes carry a step's difference on: held two orders tighter beside FP64 nuclei

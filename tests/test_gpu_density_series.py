@@ -59,3 +59,30 @@ def test_other_sub_step_counts_keep_tsit5(nsub):
     err = np.abs(_run(2, 4.0, 10, r0, v0, sig0, 0, nsub)[2] - ref).max()
     lo, hi = {1: (1e-5, 1e-1), 4: (1e-9, 1e-5), 6: (1e-10, 1e-6)}[nsub]
     assert lo < err < hi
+
+
+@pytest.mark.parametrize("coupling", [0.0, 1e-150, 3e-141, 1e-12, 0.005, 0.3])
+def test_two_state_eigenvectors(oracle, coupling):
+    """From exactly degenerate diabats to strong coupling: splittings whose square leaves the range of a double take
+    the square roots themselves.  Two steps from rest at and around the crossing, so that every lane keeps its splitting.
+    FP64 coordinates only: in FP32 the model itself is degenerate within 1e-8 of the crossing."""
+    from nqcd_mi355x import _lib as L
+    p = [0.01, 1.6, coupling, 1.0]
+    r0 = np.array([0.0, 0.0, 1e-15, -1e-9, 1e-3, -0.4, 2.0, -3.0])[:, None]
+    sig0 = np.zeros((8, 2, 2), complex)
+    sig0[:, 0, 0], sig0[:, 1, 1] = 0.75, 0.25
+    E = L.Ensemble(0)
+    E.set_problem(L.METHOD_EHRENFEST, 2, 1, 1, [MASS], 0.1)
+    E.set_model(0, 0, p)
+    E.load_initial(r0, np.zeros((8, 1)), sig0)
+    E.run(0.0, 0.2, 1)
+    r, v = E.download(L.FIELD_R), E.download(L.FIELD_V)
+    E.close()
+    c = oracle.run_ensemble(1, oracle.make_model(0, 2, 1, p), MASS, r0, np.zeros((8, 1)), sig0, dt=0.1, nsteps=2, key=1)
+    # a coupling of 1e-150 at the crossing itself: the derivative coupling's square overflows, here and there alike
+    bad = np.isnan(c["v"])
+    assert np.array_equal(np.isnan(v), bad) and np.array_equal(np.isnan(r), np.isnan(c["r"]))
+    assert coupling in (0.0, 1e-150, 3e-141) or not bad.any()
+    # accelerations of at most 0.016 / 2000 over 0.2, velocities of 1.6e-6, to 1e-12 of that: a dozen roundings make 3e-15
+    assert np.nanmax(np.abs(v - c["v"])) < 1.6e-18
+    assert np.nanmax(np.abs(r - c["r"])) < 1e-15   # positions of 3 rounded twice
