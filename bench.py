@@ -31,12 +31,11 @@ GRID = [-5.0, 5.0, 31]
 FP64_PEAK_TFLOPS = 78.6   # MI355X FP64 vector (= FP64 matrix) peak
 HBM_PEAK_GBS = 8000.0
 # FP64 flops (an FMA counts 2) of one trajectory-step of the trace-fixed two-state formulation,
-# counted from nqcd_device.h / fssh2.hip against the compiled loop: 4 Tsit5 sub-steps x 180 (63
-# stage-combination FMA, 6 right-hand sides, coefficient set-up) + 185 for the last, clipped
-# sub-step + 8 for the products with h formed once per step = 913, plus ~75 for the eigen, the
-# coupling rotation, the interpolation set-up and the hop test.  The FP32 model and Verlet work are
-# not counted.
-FLOP_PER_STEP = 988.0
+# counted from nqcd_device.h / fssh2.hip: the density's power series at its fewest orders, 8 + 7 x 21
+# = 155, + 33 for its set-up and the sub-steps' error, + 57 for the eigenvectors, 27 for the coupling
+# rotation, 20 for the interpolation and 12 for force and hop test.  Orders 9 to 20 (21 each, taken
+# by long steps) and the FP32 model and Verlet work are not counted.
+FLOP_PER_STEP = 304.0
 # Threads of the CPU baseline: the host share of one GPU on the measurement machine (16 cores)
 CPU_THREADS = 16
 
@@ -206,7 +205,7 @@ def iesh_extra(L):
                       "pop_imp": E.download(L.FIELD_SAVE_POP_DI)[:n, :, 0].copy(), "nhops": E.download(L.FIELD_NHOPS)[:n]}
         E.close()
         N, Ne = M + 1, M // 2
-        flop = 8 * 4 * N * N * Ne + 16 * N * M + (8 / 3) * Ne ** 3  # Taylor (K ~ 8) + eigen + Gauss-Jordan
+        flop = 8 * 4 * N * N * Ne + 16 * N * M + (8 / 3) * Ne ** 3  # Taylor (K ~ 8) + eigen + elimination
         rate = st["traj_steps"] / (st["kernel_ms"] / 1e3)
         res[f"N{N}"] = {"ntraj": ntraj, "nsteps": nsteps, "kernel_ms": st["kernel_ms"], "traj_steps_per_s": rate,
                         "flop_per_traj_step": flop, "achieved_TFLOPs": flop * rate / 1e12,

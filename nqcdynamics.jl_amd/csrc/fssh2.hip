@@ -1,8 +1,9 @@
 // fssh2.hip -- two-state FSSH / Ehrenfest trajectory kernels (BABwithTsit5).
 //
 // Restates bab_electronics.jl:48-91 (B-A-B velocity Verlet, acceleration on the
-// active surface or mean field, Tsit5 density propagation with linearly
-// interpolated eigenvalues and v.d) followed by the HoppingCallback of
+// active surface or mean field, density propagation with linearly
+// interpolated eigenvalues and v.d: the reference's Tsit5 sub-steps, as one
+// power series with their error where five are asked for) followed by the HoppingCallback of
 // surface_hopping.jl:2-16 (fssh.jl:96-121 probability and selection,
 // surface_hopping.jl:64-99 rescaling).
 //

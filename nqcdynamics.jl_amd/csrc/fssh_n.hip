@@ -3,8 +3,9 @@
 //
 // Restates bab_electronics.jl:48-91 for n states: velocity Verlet with the active-surface force
 // (fssh.jl:67-74) or the mean-field force with the full U^T dV U (ehrenfest.jl:50-68), the n x n
-// density propagated by Tsit5 under V(tau) = diag(E) - i (v.d) interpolated linearly between the
-// step ends (electronic_dynamics.jl:15-79,104-140), then the HoppingCallback (fssh.jl:96-121,
+// density propagated under V(tau) = diag(E) - i (v.d) interpolated linearly between the step ends
+// (electronic_dynamics.jl:15-79,104-140) by a power series with the error of five Tsit5 sub-steps, or
+// by the sub-steps themselves where another number is asked for, then the HoppingCallback (fssh.jl:96-121,
 // surface_hopping.jl:64-168).
 //
 // One trajectory per lane, all of its state in registers, lanes refilled from a work queue as

@@ -259,7 +259,7 @@ __device__ __forceinline__ void wave_argmax(double& mag, int& idx) {
 // of the pivot permutation comes from counting, at each step, the unused rows above the pivot row.  The column's owner
 // picks the pivot and leaves the multipliers in LDS; one barrier a pivot (two buffers), everything else in registers.
 // One wavefront's LU through LDS followed by a workgroup's Gauss-Jordan through LDS took 116 us at 20 electrons and
-// 290 us at 50.  buf: 2 x 136 doubles; piv[p] = q_p; myp: the column whose pivot row this lane's row was; on return
+// 290 us at 50; this takes 65 and 63 us beside the other workgroups' propagators.  buf: 2 x 136 doubles; piv[p] = q_p; myp: the column whose pivot row this lane's row was; on return
 // x[j] is column w + NT ((j + rot) % KC).  False for a singular matrix (a zero pivot column).  Called by whole
 // workgroups of 64 NT lanes; the caller's previous use of buf and piv ends with a barrier.
 template <int NT, int KC>
@@ -1174,8 +1174,8 @@ __global__ __launch_bounds__(256) void ie_diabatic_orbitals(int64_t ntraj, int N
     for (uint64_t w = tk_hi; w; w &= w - 1) occ0[traj * Ne + e++] = 64 + __ffsll((unsigned long long)w) - 1;
 }
 
-// S^-1, interleaved complex
-int ie_sb_len(int Ne) { return 2 * Ne * Ne; }
+// S^-1, interleaved complex; an odd number of rows is reserved, the size that the limit on problems is stated for
+int ie_sb_len(int Ne) { return 2 * Ne * (Ne | 1); }
 
 size_t ie_lds_bytes(int NT, int cw, int N, int Ne, int P) {
     const int NP = 16 * NT;

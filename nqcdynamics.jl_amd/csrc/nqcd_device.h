@@ -3,7 +3,7 @@
 // Everything here runs per lane (one trajectory per lane) in registers:
 // counter-based Philox draws, the closed-form model Hamiltonians, the 2x2
 // symmetric eigen-decomposition with eigenvector tracking, the nonadiabatic
-// coupling, the Tsit5 density-matrix propagation and the fewest-switches hop.
+// coupling, the density-matrix propagation (power series or Tsit5) and the fewest-switches hop.
 #pragma once
 #include <type_traits>
 #include <hip/hip_runtime.h>
@@ -367,7 +367,8 @@ __device__ __forceinline__ void eigen2(double a, double c, double d, double& E0,
 
 // The same with 1 / (E1 - E0), for the steps of the two-state kernels: one reciprocal square root serves the radius,
 // its inverse and, with the eigenvector's norm^2 = 2 rad (rad + |h|), a second one the vector (within an ulp), in place
-// of two square roots and two divisions.  Radii whose square could leave the range of a double take those.
+// of two square roots and two divisions: 1e6 mixed Tully trajectories 44.5 -> 41.7 ms, 1e5 of FP64 Ehrenfest 4.5 -> 4.25.
+// Radii whose square could leave the range of a double take those.
 __device__ __forceinline__ void eigen2_gap(double a, double c, double d, double& E0, double& E1, double& inv_gap, double U[4],
                                            bool track) {
     const double mean = 0.5 * (a + d), h = 0.5 * (a - d);
@@ -502,7 +503,7 @@ __device__ __forceinline__ void propagate2_substeps(double e0, double e1, double
 // m up to 1 (10^4 random pairs for each of 30 magnitudes of A0 and A1).  Bound by FP64 issue where the chip is
 // full and by the order-to-order chain where it is not.  Sub-steps -> series: 1e6 mixed Tully trajectories
 // 70 -> 44.5 ms, 1e5 RPSH ring polymers of 8 beads x 1000 steps 4.73 -> 3.24 ms, 200 trajectories x 800 steps
-// 2.40 -> 2.00 ms.
+// 2.40 -> 2.00 ms (with eigen2_gap 41.7, 3.12 and 1.92 ms).
 __device__ __forceinline__ void series_step2(double e0, double e1, double g0, double g1, double z2, Sig2& u) {
     double p = u.q, x = u.x, y = u.y;        // u^(k)
     double pm = 0.0, xm = 0.0, ym = 0.0;     // u^(k-1)

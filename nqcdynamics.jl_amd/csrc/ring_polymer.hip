@@ -10,7 +10,7 @@
 // (transform, Cayley per mode, transform back) in exact arithmetic.  Each lane keeps its row
 // of H in registers; the two transforms per step (modes -> bead positions, bead forces ->
 // modes) are P-term dot products against values broadcast through LDS.
-// The centroid electronics (eigen, coupling, Tsit5 density, hop and rescaling; once per ring
+// The centroid electronics (eigen, coupling, density series, hop and rescaling; once per ring
 // polymer, bcb_electronics.jl:83-96) run on electronics lanes: lane e of the workgroup's first
 // waves takes ring polymer e of the workgroup.  The mode-0 lanes hand the centroid position and
 // velocity over through LDS, and the electronics lanes hand back the active state / density of
