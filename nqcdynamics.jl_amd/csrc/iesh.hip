@@ -488,7 +488,9 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(NT <= 4
             return s;
         };
         // acceleration at the eigenpairs whose impurity components are Uv, with the wavefunction in Tb
-        // (iesh.jl:190-207, ehrenfest_na.jl:72-86; per bead rpiesh.jl:20-38, rpehrenfest_na.jl:14-40)
+        // (iesh.jl:190-207, ehrenfest_na.jl:72-86; per bead rpiesh.jl:20-38, rpehrenfest_na.jl:14-40).  Ends without a
+        // barrier: pcol (EhrenfestNA), occ, Uv and Tb are still being read, and the caller puts a workgroup barrier
+        // before the next write to any of them.
         auto accel = [&](const Scalars& s, const double* Uv) -> double {
             IE_IDS
             // summed by every wavefront for itself (Ne <= 64)
@@ -608,8 +610,8 @@ __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(NT <= 4
         double kacc = 0.0;
         if (rp) bead_accels();
         else kacc = accel(sc, U);
+        __syncthreads();  // accel's reads of pcol end here, before save writes it
         save(0);
-        __syncthreads();
 
         for (int64_t step = 0; step < A.nsteps; ++step) {
             if (!rp) {
