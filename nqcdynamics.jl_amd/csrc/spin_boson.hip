@@ -102,7 +102,8 @@ __device__ __forceinline__ SbTab<R> sb_here(SbTab<R> p) {
 // A step is two passes over the modes with the electronics between them.  Both half kicks that meet at a step
 // end see the same positions and the same force factor F (the acceleration of the step end stands, also after a
 // hop), so one pass applies them together: v = u - a is the velocity at the step end, whose projection on c the
-// coupling needs, and u' = 2 v - u the one after the next step's first half kick.
+// coupling needs, and u' = u - 2 a the one after the next step's first half kick.  The kick a is formed first, so
+// that a velocity is rounded at its own size once a step (velocity Verlet step by step rounds it twice).
 //
 // The positions of the last NL modes stay in LDS ([chunk][lane], 16 bytes a lane and access), the rest and all
 // velocities in registers: with all 2 NB values in registers a wavefront took 352 registers, so the 1,563
@@ -262,10 +263,10 @@ __device__ __forceinline__ void sb_body(const SbArgs* __restrict__ Ap, SbVec<R>*
                     const SbVec<R> xq = q < NCR ? load_x(q) : xa[cur][i];
 #pragma unroll
                     for (int k = 0; k < 4; ++k) {                    // step_B! twice
-                        const R vn = v[4 * q + k] - c[cur][i][0][k] * xq[k] - c[cur][i][1][k] * Fn;
-                        Vc += c[cur][i][2][k] * vn;
-                        v[4 * q + k] = (R)2 * vn - v[4 * q + k];
-                        asm volatile("" : "+v"(v[4 * q + k]));   // formed here: left to be sunk, vn and the old v both live on
+                        const R a = c[cur][i][0][k] * xq[k] + c[cur][i][1][k] * Fn;
+                        Vc += c[cur][i][2][k] * (v[4 * q + k] - a);
+                        v[4 * q + k] = v[4 * q + k] - (R)2 * a;
+                        asm volatile("" : "+v"(v[4 * q + k]));   // formed here: left to be sunk, a and the old v both live on
                     }
                 }
                 __builtin_amdgcn_sched_barrier(0);
