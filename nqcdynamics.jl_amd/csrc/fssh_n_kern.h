@@ -642,7 +642,7 @@ __device__ __forceinline__ void ns_step(const FsshNArgs* Ap, const FsshNArgs& A,
             w1[p] = (H.dt * len) * d1;
         }
         const double m0 = ns_norm<NM>(L.n, e0, w0), m1 = ns_norm<NM>(L.n, e1, w1);
-        const double z2 = fma(4.0, m1, m0 * m0);
+        double z2 = fma(4.0, m1, m0 * m0);
         int parts = 1;
         if constexpr (sizeof(R) == 8) {
             // FP64 nuclei: where the sub-steps' own error and theirs on the change of A stay below 1e-12 a step
@@ -650,8 +650,14 @@ __device__ __forceinline__ void ns_step(const FsshNArgs* Ap, const FsshNArgs& A,
             const double m = m0 + m1, mm = m * m;
             series = 1.4e-8 * (mm * mm) * (mm + m1) < 1e-12;
         } else {
-            // FP32 nuclei: the series throughout, on parts of the step beyond z2 = 4
-            if (z2 >= 4.0) parts = (int)fmin(ceil(0.5 * sqrt(z2)), 64.0);
+            // FP32 nuclei: the series throughout, on parts of the step beyond z2 = 4.  A later part starts from what the
+            // generator has grown to, at most m0 + m1, so parts and orders follow from that.  The 64 parts serve norms
+            // up to 126; beyond them no accuracy is promised, as with five sub-steps at such norms.
+            if (z2 >= 4.0) {
+                const double m = m0 + m1;
+                z2 = fma(4.0, m1, m * m);
+                parts = (int)fmin(ceil(0.5 * sqrt(z2)), 64.0);
+            }
         }
         if (series) {
             if constexpr (sizeof(R) == 8) {
