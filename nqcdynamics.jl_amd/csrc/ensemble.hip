@@ -302,8 +302,11 @@ hipError_t launch_zero(void* p, size_t bytes, hipStream_t s) {
 // rows both move whole segments, into a bounded staging buffer that is copied straight into the caller's array:
 // bound by the copy to the host.  1e5 ring polymers of 32 beads, 1000 steps and their final positions: 10.1 ms with a
 // copy into a host vector and a strided host pass, 4.5 ms here (2.5 of them the steps).
+// Workgroups take 64 trajectories (x) and every gridDim.y-th tile of rows: with few trajectories the rows have to fill
+// the chip (a tile of one workgroup's walk is a memory round trip: 2e5 rows of one trajectory took 10 ms).
 // ---------------------------------------------------------------------------
 constexpr int kTileT = 64, kTileR = 16;
+constexpr int64_t kTileGroups = 4096;   // workgroups beyond which rows are walked and not spread
 // Output row k is source row (k / g) * G + k % g.
 template <typename T>
 __global__ __launch_bounds__(256) void transpose_rows(const T* __restrict__ src, int64_t nt, int32_t g, int32_t G,
@@ -312,7 +315,8 @@ __global__ __launch_bounds__(256) void transpose_rows(const T* __restrict__ src,
     const int64_t tb = (int64_t)blockIdx.x * kTileT;
     const int tl = threadIdx.x & 63, rl = threadIdx.x >> 6;
     const int rw = threadIdx.x & 15, tw = threadIdx.x >> 4;
-    for (int32_t rb = 0; rb < rows; rb += kTileR) {
+    for (int64_t rt = blockIdx.y; rt * kTileR < rows; rt += gridDim.y) {
+        const int32_t rb = (int32_t)(rt * kTileR);
 #pragma unroll
         for (int k = 0; k < kTileR; k += 4) {
             const int32_t r = rb + rl + k;
@@ -369,14 +373,16 @@ static int32_t download_rows_t(nqcd_handle_t* h, const DevBuf& b, int32_t first,
     const size_t end = (size_t)first + (size_t)((rows - 1) / g) * G + (rows - 1) % g + 1;
     if (!b.p || b.bytes < sizeof(T) * end * (size_t)h->ntraj) return fail(h, NQCD_ERR_STATE, "this run kept no such field");
     const T* src = b.as<T>() + (size_t)first * h->ntraj;
-    if (rows == 1) {
-        HIPCHK(h, hipMemcpyAsync(out, src, sizeof(T) * (size_t)h->ntraj, hipMemcpyDeviceToHost, h->stream));
+    if (rows == 1 || (h->ntraj == 1 && (g == G || rows <= g))) {   // in the caller's order already
+        HIPCHK(h, hipMemcpyAsync(out, src, sizeof(T) * (size_t)rows * (size_t)h->ntraj, hipMemcpyDeviceToHost, h->stream));
         HIPCHK(h, hipStreamSynchronize(h->stream));
         return NQCD_OK;
     }
     return download_chunks(h, sizeof(T) * (size_t)rows, out, [&](int64_t t0, int64_t cnt, void* stage) {
-        hipLaunchKernelGGL(transpose_rows<T>, dim3((unsigned)((cnt + kTileT - 1) / kTileT)), dim3(256), 0, h->stream, src,
-                           h->ntraj, g, G, rows, t0, cnt, static_cast<T*>(stage));
+        const int64_t gx = (cnt + kTileT - 1) / kTileT, tiles = ((int64_t)rows + kTileR - 1) / kTileR;
+        const int64_t gy = std::min(tiles, std::max<int64_t>(kTileGroups / gx, 1));
+        hipLaunchKernelGGL(transpose_rows<T>, dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, h->stream, src, h->ntraj, g, G,
+                           rows, t0, cnt, static_cast<T*>(stage));
     });
 }
 
