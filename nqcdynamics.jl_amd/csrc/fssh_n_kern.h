@@ -294,10 +294,20 @@ __device__ __forceinline__ void ns_rhs(const double e[NM], const double w[], con
 }
 
 // 1 / k!, read with scalar loads by the rolled series
-__constant__ double kInvFactorial[21] = {1.0, 1.0, 1.0 / 2.0, 1.0 / 6.0, 1.0 / 24.0, 1.0 / 120.0, 1.0 / 720.0, 1.0 / 5040.0,
-    1.0 / 40320.0, 1.0 / 362880.0, 1.0 / 3628800.0, 1.0 / 39916800.0, 1.0 / 479001600.0, 1.0 / 6227020800.0,
-    1.0 / 87178291200.0, 1.0 / 1307674368000.0, 1.0 / 20922789888000.0, 1.0 / 355687428096000.0, 1.0 / 6402373705728000.0,
-    1.0 / 121645100408832000.0, 1.0 / 2432902008176640000.0};
+constexpr int kNsMaxOrders = 63;
+struct InvFactorials {
+    double v[kNsMaxOrders + 1];
+};
+constexpr InvFactorials ns_inv_factorials() {
+    InvFactorials t{};
+    long double f = 1.0L;
+    for (int k = 0; k <= kNsMaxOrders; ++k) {
+        if (k > 1) f *= k;
+        t.v[k] = (double)(1.0L / f);
+    }
+    return t;
+}
+__constant__ InvFactorials kInvFactorial = ns_inv_factorials();
 
 // The density over a nuclear step as one power series (series_step2 in nqcd_device.h, for the n-state equation):
 // over the step the energies and couplings are e + e1 s, w + w1 s for s in [0, 1] (times dt), so the derivatives
@@ -308,6 +318,19 @@ __constant__ double kInvFactorial[21] = {1.0, 1.0, 1.0 / 2.0, 1.0 / 6.0, 1.0 / 2
 // trajectories x 1000 steps, with the cheaper Jacobi rotations and the tables in LDS: 20.8 -> 8.9 ms).
 __device__ __forceinline__ int ns_series_orders(double z2) {
     return z2 > 0.0041 ? (z2 > 0.022 ? (z2 > 0.075 ? (z2 > 0.19 ? (z2 > 0.35 ? (z2 > 0.65 ? 20 : 18) : 16) : 14) : 12) : 10) : 8;
+}
+
+// Orders of each of `parts` equal parts of a step whose generator starts at a norm of m - m1 and changes by m1 (z2 >= 4,
+// FP32 nuclei; rp = 1 / parts).  A later part starts from what the generator has grown to, so each is taken to start
+// from m / parts, and z bounds the norm at its end.  The count leaves less than 1e-10 of the majorant series (computed
+// for z from 2 to 12 and every share of m1 in it); at z = 12 its cancellation costs 2e-11.  Few long parts: a unit
+// of z takes about three orders where parts of z = 2 take ten (100 steps of 1e5 three-state trajectories, at a norm of 6:
+// 3.9 -> 2.0 ms, at 25: 10.2 -> 5.1; five sub-steps: 2.3 ms, off by 7e-4 a step at 6 and unstable at 25).  Beyond a
+// norm of 500 to 760, where the 64 parts end, no accuracy is promised.
+__device__ __forceinline__ int ns_long_orders(int parts, double rp, double m, double m1) {
+    const double z = parts > 1 ? rp * fma(rp, m1, m) : m;
+    const double share = (parts > 1 ? rp * rp * m1 : m1) / z;
+    return (int)fmin(fma(3.2, z, 14.0) + 11.0 * sqrt(share), (double)kNsMaxOrders);
 }
 
 template <int NM>
@@ -335,7 +358,7 @@ __device__ __forceinline__ void ns_series(const double e[NM], const double w[], 
     for (int p = 0; p < NP; ++p) { kx[p] = x[p]; ky[p] = y[p]; px[p] = 0.0; py[p] = 0.0; wk[p] = 0.0; }
 #pragma unroll 1
     for (int k = 1; k <= orders; ++k) {
-        const double rf = kInvFactorial[k];
+        const double rf = kInvFactorial.v[k];
         double fa[NM], fx[NQ], fy[NQ];
         ns_rhs<NM, false>(ek, wk, pa, px, py, fa, fx, fy);
         ns_rhs<NM, true>(e, w, ka, kx, ky, fa, fx, fy);
@@ -642,7 +665,7 @@ __device__ __forceinline__ void ns_step(const FsshNArgs* Ap, const FsshNArgs& A,
             w1[p] = (H.dt * len) * d1;
         }
         const double m0 = ns_norm<NM>(L.n, e0, w0), m1 = ns_norm<NM>(L.n, e1, w1);
-        double z2 = fma(4.0, m1, m0 * m0);
+        const double z2 = fma(4.0, m1, m0 * m0);
         int parts = 1;
         if constexpr (sizeof(R) == 8) {
             // FP64 nuclei: where the sub-steps' own error and theirs on the change of A stay below 1e-12 a step
@@ -650,21 +673,15 @@ __device__ __forceinline__ void ns_step(const FsshNArgs* Ap, const FsshNArgs& A,
             const double m = m0 + m1, mm = m * m;
             series = 1.4e-8 * (mm * mm) * (mm + m1) < 1e-12;
         } else {
-            // FP32 nuclei: the series throughout, on parts of the step beyond z2 = 4.  A later part starts from what the
-            // generator has grown to, at most m0 + m1, so parts and orders follow from that.  The 64 parts serve norms
-            // up to 126; beyond them no accuracy is promised, as with five sub-steps at such norms.
-            if (z2 >= 4.0) {
-                const double m = m0 + m1;
-                z2 = fma(4.0, m1, m * m);
-                parts = (int)fmin(ceil(0.5 * sqrt(z2)), 64.0);
-            }
+            // FP32 nuclei: the series throughout, on parts of a step whose generator passes a norm of 12
+            if (z2 >= 4.0) parts = (int)fmin(ceil(fma(0.5, m1, m0 + m1) * (1.0 / 12.0)), 64.0);
         }
         if (series) {
             if constexpr (sizeof(R) == 8) {
                 ns_series<NM>(e0, w0, e1, w1, ns_series_orders(z2), L.a, L.x, L.y);
             } else {
                 const double rp = nr_rcp((double)parts);
-                const int orders = ns_series_orders(z2 * rp * rp);
+                const int orders = z2 >= 4.0 ? ns_long_orders(parts, rp, m0 + m1, m1) : ns_series_orders(z2);
 #pragma unroll
                 for (int i = 0; i < NM; ++i) { e0[i] *= rp; e1[i] *= rp * rp; }
 #pragma unroll
