@@ -307,10 +307,9 @@ hipError_t launch_zero(void* p, size_t bytes, hipStream_t s) {
 // ---------------------------------------------------------------------------
 constexpr int kTileT = 64, kTileR = 16;
 constexpr int64_t kTileGroups = 4096;   // workgroups beyond which rows are walked and not spread
-// Output row k is source row (k / g) * G + k % g.
 template <typename T>
-__global__ __launch_bounds__(256) void transpose_rows(const T* __restrict__ src, int64_t nt, int32_t g, int32_t G,
-                                                      int32_t rows, int64_t t0, int64_t cnt, T* __restrict__ out) {
+__global__ __launch_bounds__(256) void transpose_rows(const T* __restrict__ src, int64_t nt, int32_t rows, int64_t t0,
+                                                      int64_t cnt, T* __restrict__ out) {
     __shared__ T tile[kTileR][kTileT + 1];
     const int64_t tb = (int64_t)blockIdx.x * kTileT;
     const int tl = threadIdx.x & 63, rl = threadIdx.x >> 6;
@@ -320,7 +319,7 @@ __global__ __launch_bounds__(256) void transpose_rows(const T* __restrict__ src,
 #pragma unroll
         for (int k = 0; k < kTileR; k += 4) {
             const int32_t r = rb + rl + k;
-            if (r < rows && tb + tl < cnt) tile[rl + k][tl] = src[((int64_t)(r / g) * G + r % g) * nt + t0 + tb + tl];
+            if (r < rows && tb + tl < cnt) tile[rl + k][tl] = src[r * nt + t0 + tb + tl];
         }
         __syncthreads();
 #pragma unroll
@@ -368,12 +367,12 @@ static int32_t download_chunks(nqcd_handle_t* h, size_t row_bytes, void* out, F&
 }
 
 template <typename T>
-static int32_t download_rows_t(nqcd_handle_t* h, const DevBuf& b, int32_t first, int32_t g, int32_t G, int32_t rows, T* out) {
+static int32_t download_rows_t(nqcd_handle_t* h, const DevBuf& b, int32_t first, int32_t rows, T* out) {
     if (rows <= 0 || h->ntraj <= 0) return NQCD_OK;
-    const size_t end = (size_t)first + (size_t)((rows - 1) / g) * G + (rows - 1) % g + 1;
-    if (!b.p || b.bytes < sizeof(T) * end * (size_t)h->ntraj) return fail(h, NQCD_ERR_STATE, "this run kept no such field");
+    if (!b.p || b.bytes < sizeof(T) * ((size_t)first + rows) * (size_t)h->ntraj)
+        return fail(h, NQCD_ERR_STATE, "this run kept no such field");
     const T* src = b.as<T>() + (size_t)first * h->ntraj;
-    if (rows == 1 || (h->ntraj == 1 && (g == G || rows <= g))) {   // in the caller's order already
+    if (rows == 1 || h->ntraj == 1) {   // in the caller's order already
         HIPCHK(h, hipMemcpyAsync(out, src, sizeof(T) * (size_t)rows * (size_t)h->ntraj, hipMemcpyDeviceToHost, h->stream));
         HIPCHK(h, hipStreamSynchronize(h->stream));
         return NQCD_OK;
@@ -381,19 +380,16 @@ static int32_t download_rows_t(nqcd_handle_t* h, const DevBuf& b, int32_t first,
     return download_chunks(h, sizeof(T) * (size_t)rows, out, [&](int64_t t0, int64_t cnt, void* stage) {
         const int64_t gx = (cnt + kTileT - 1) / kTileT, tiles = ((int64_t)rows + kTileR - 1) / kTileR;
         const int64_t gy = std::min(tiles, std::max<int64_t>(kTileGroups / gx, 1));
-        hipLaunchKernelGGL(transpose_rows<T>, dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, h->stream, src, h->ntraj, g, G,
-                           rows, t0, cnt, static_cast<T*>(stage));
+        hipLaunchKernelGGL(transpose_rows<T>, dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, h->stream, src, h->ntraj, rows,
+                           t0, cnt, static_cast<T*>(stage));
     });
 }
 
 int32_t download_rows(nqcd_handle_t* h, const DevBuf& src, int32_t first, int32_t rows, double* out) {
-    return download_rows_t<double>(h, src, first, rows, rows, rows, out);
+    return download_rows_t<double>(h, src, first, rows, out);
 }
 int32_t download_rows(nqcd_handle_t* h, const DevBuf& src, int32_t first, int32_t rows, int32_t* out) {
-    return download_rows_t<int32_t>(h, src, first, rows, rows, rows, out);
-}
-int32_t download_row_groups(nqcd_handle_t* h, const DevBuf& src, int32_t first, int32_t g, int32_t G, int32_t rows, double* out) {
-    return download_rows_t<double>(h, src, first, g, G, rows, out);
+    return download_rows_t<int32_t>(h, src, first, rows, out);
 }
 int32_t download_density2(nqcd_handle_t* h, bool im, double* out) {
     if (h->ntraj <= 0) return NQCD_OK;

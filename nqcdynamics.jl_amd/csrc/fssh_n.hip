@@ -273,7 +273,7 @@ int32_t ns_run(nqcd_handle_t* h, double t0, int64_t nsteps, const nqcd_term_desc
 }
 
 int32_t ns_download(nqcd_handle_t* h, int32_t field, void* out, int64_t bytes) {
-    const int n = h->prob.n_states, NM = ns_kernel_states(n);
+    const int n = h->prob.n_states;   // the kernel's count as well
     const int64_t nt = h->ntraj;
     const int ns = h->nsave;
     auto need = [&](int64_t b) -> int32_t {
@@ -289,8 +289,7 @@ int32_t ns_download(nqcd_handle_t* h, int32_t field, void* out, int64_t bytes) {
     case NQCD_FIELD_SIGMA_RE:
     case NQCD_FIELD_SIGMA_IM: {
         if (int32_t rc = need(8 * (int64_t)n * n * nt)) return rc;
-        return download_row_groups(h, h->sig, field == NQCD_FIELD_SIGMA_IM ? NM * NM : 0, n, NM, n * n,
-                                   static_cast<double*>(out));
+        return download_rows(h, h->sig, field == NQCD_FIELD_SIGMA_IM ? n * n : 0, n * n, static_cast<double*>(out));
     }
     case NQCD_FIELD_STATE:
     case NQCD_FIELD_STEPS:
@@ -303,8 +302,7 @@ int32_t ns_download(nqcd_handle_t* h, int32_t field, void* out, int64_t bytes) {
     case NQCD_FIELD_SAVE_POP_AD:
     case NQCD_FIELD_SAVE_POP_DI: {
         if (int32_t rc = need(8 * (int64_t)n * ns * nt)) return rc;
-        return download_row_groups(h, field == NQCD_FIELD_SAVE_POP_AD ? h->save_ad : h->save_di, 0, n, NM, n * ns,
-                                   static_cast<double*>(out));
+        return download_rows(h, field == NQCD_FIELD_SAVE_POP_AD ? h->save_ad : h->save_di, 0, n * ns, static_cast<double*>(out));
     }
     case NQCD_FIELD_SAVE_STATE: {
         if (int32_t rc = need(4 * (int64_t)ns * nt)) return rc;

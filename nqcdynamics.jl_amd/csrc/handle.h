@@ -31,12 +31,11 @@ struct DevBuf {
 
 int32_t fail(nqcd_handle_t* h, int32_t code, const std::string& msg);
 
-// Per-trajectory fields to the host: `rows` device rows [row][trajectory] from row `first` on as [trajectory][row] (ensemble.hip); of a
-// group of G device rows, the first g (n-state kernels of more states than the problem); the two-state densities.
-constexpr size_t kStageBytes = size_t(64) << 20;   // most of the staging buffer a handle keeps for these
+// Per-trajectory fields to the host: `rows` device rows [row][trajectory] from row `first` on as [trajectory][row]
+// (ensemble.hip); the two-state densities.
+constexpr size_t kStageBytes = size_t(64) << 20;   // the staging buffer a handle keeps for these, at most (or one trajectory's field)
 int32_t download_rows(nqcd_handle_t* h, const DevBuf& src, int32_t first, int32_t rows, double* out);
 int32_t download_rows(nqcd_handle_t* h, const DevBuf& src, int32_t first, int32_t rows, int32_t* out);
-int32_t download_row_groups(nqcd_handle_t* h, const DevBuf& src, int32_t first, int32_t g, int32_t G, int32_t rows, double* out);
 int32_t download_density2(nqcd_handle_t* h, bool im, double* out);
 
 }  // namespace nqcd

@@ -36,7 +36,7 @@ def test_rows(P, ntraj):
 @pytest.mark.parametrize("n", [2, 3, 5, 8])
 @pytest.mark.parametrize("ntraj", [1, 64, 129])
 def test_density(n, ntraj):
-    """States the kernel has and the problem has not (n = 5) leave gaps between the rows."""
+    """The n-state densities, whose imaginary parts lie behind the real ones."""
     from nqcd_mi355x import _lib as L
     rng = np.random.default_rng(n)
     s = rng.normal(size=(ntraj, n, n)) + 1j * rng.normal(size=(ntraj, n, n))
