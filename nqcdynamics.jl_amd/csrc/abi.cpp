@@ -69,6 +69,30 @@ int64_t nqcd_rows(const nqcd_handle* h) { return (int64_t)h->D * (is_rp(h) ? h->
 
 int nsub_of(const nqcd_handle* h) { return h->prob.electronic_substeps > 0 ? h->prob.electronic_substeps : 5; }
 
+// Upper bound of a two-state model's adiabatic gap, sqrt((V11 - V22)^2 + 4 V12^2), from its parameters.
+double gap_bound(const ModelSlot& m) {
+    const double* p = m.p;
+    switch (m.kind) {
+    case NQCD_MODEL_TULLY1: return 2.0 * std::hypot(p[0], p[2]);
+    case NQCD_MODEL_TULLY2: return std::hypot(std::max(std::fabs(p[4]), std::fabs(p[4] - p[0])), 2.0 * p[2]);
+    case NQCD_MODEL_TULLY3: return 2.0 * std::hypot(p[0], 2.0 * p[1]);
+    default: return std::hypot(p[2], 2.0 * p[3]);   // the double well with its Gaussian coupling
+    }
+}
+
+// Whether a launch takes the density's power series.  Five sub-steps, and a step short enough for the models' largest
+// gap: beyond gap x dt = 0.45 (FP64 nuclei) and 1.9 (FP32) so many lanes are past the series' own limits (propagate2)
+// that most wavefronts would pay for both forms.  2e5 FSSH trajectories on Tully's models 1 / 2 / 3, sub-steps alone over
+// series where it serves: FP64 1.27 / 1.49 / 1.53 at gap x dt = 0.15, 0.90 / 0.93 / 1.47 at 0.4, 0.84 / 0.86 / 0.97 at 0.65,
+// 0.86 / 0.94 / 0.93 at 1; FP32 1.10 / 1.18 / 1.33 at 1.6, 1.10 / 0.85 / 0.89 at 2.5.
+bool series_serves(const nqcd_handle* h) {
+    if (nsub_of(h) != 5) return false;
+    double gap = 0.0;
+    for (int m = 0; m < kMaxModels; ++m)
+        if (h->model_set[m]) gap = std::max(gap, gap_bound(h->models[m]));
+    return gap * h->prob.dt < (h->prob.precision == NQCD_PREC_FP64 ? 0.45 : 1.9);
+}
+
 // Queue order: stable grouping by model so a wavefront refills with one model.
 std::vector<int32_t> order_by_model(const std::vector<int32_t>& mid, int64_t ntraj) {
     std::vector<int32_t> ord(ntraj);
@@ -114,6 +138,7 @@ Fssh2Args make_args(nqcd_handle* h, double t0, int64_t nsteps, const nqcd_term_d
     A.method = (h->prob.method == NQCD_METHOD_FSSH) ? METHOD_FSSH : METHOD_EHRENFEST;
     A.rescaling = h->prob.rescaling;
     A.nsub = nsub_of(h);
+    A.series = series_serves(h);
     A.save_every = h->save_every;
     A.nsave = h->nsave;
     A.term_kind = term ? term->kind : 0;

@@ -38,6 +38,7 @@ struct Fssh2Args {
     int64_t ntraj;
     int32_t method, rescaling, nsub, save_every;
     int32_t nsave, term_kind, term_dof, nmodels;
+    int32_t series, pad;        // series: the density by the power series where it serves
     double term_value, dt, t0;
     int64_t nsteps;
     uint64_t key;

@@ -56,7 +56,7 @@ struct Lane2 {
 template <int D>
 struct Fssh2Hot {
     int32_t method, rescaling, nsub, save_every;
-    int32_t cell_mode, term_kind, term_dof, pad;
+    int32_t cell_mode, term_kind, term_dof, series;
     int64_t nsteps;
     double dt, term_value;
     uint64_t key;
@@ -69,7 +69,7 @@ __device__ __forceinline__ Fssh2Hot<D> fssh2_hot(const Fssh2Args& A) {
     H.method = uniform_sgpr(A.method); H.rescaling = uniform_sgpr(A.rescaling);
     H.nsub = uniform_sgpr(A.nsub); H.save_every = uniform_sgpr(A.save_every);
     H.cell_mode = uniform_sgpr(A.cell.mode); H.term_kind = uniform_sgpr(A.term_kind);
-    H.term_dof = uniform_sgpr(A.term_dof); H.pad = 0;
+    H.term_dof = uniform_sgpr(A.term_dof); H.series = uniform_sgpr(A.series);
     H.nsteps = uniform_sgpr(A.nsteps);
     H.dt = uniform_sgpr(A.dt); H.term_value = uniform_sgpr(A.term_value);
     H.key = uniform_sgpr(A.key);
@@ -262,7 +262,7 @@ __device__ __forceinline__ void step_traj(const Fssh2Args* Ap, const Fssh2Args& 
     const double inv = nr_rcp(tn - L.tc);
     Interp2 P;
     P.dE0 = L.dEc; P.dE1 = (dEn - L.dEc) * inv; P.w0 = L.wc; P.w1 = (w - L.wc) * inv;
-    propagate2<R>(P, L.s, L.t, L.tc, H.dt, H.nsub);
+    propagate2<R>(P, L.s, L.t, L.tc, H.dt, H.nsub, H.series != 0);
     L.dEc = dEn; L.wc = w; L.tc = tn;
     L.t = tn;
     // A save time's values are those before the step's discrete callbacks (DiffEqBase's

@@ -346,7 +346,7 @@ __device__ __forceinline__ void nd_finish_step(const FsshNdArgs* Ap, const FsshN
     const double inv = 1.0 / (tn - L.tc);
     Interp2 P;
     P.dE0 = L.dEc; P.dE1 = (dEn - L.dEc) * inv; P.w0 = L.wc; P.w1 = (w - L.wc) * inv;
-    propagate2<R>(P, L.s, L.t, L.tc, A.dt, A.nsub);
+    propagate2<R>(P, L.s, L.t, L.tc, A.dt, A.nsub, A.nsub == 5);
     L.dEc = dEn; L.wc = w; L.tc = tn;
     L.t = tn;
     // the save precedes the hop callback (a save time holds the state before the step's callbacks)

@@ -559,22 +559,22 @@ __device__ __forceinline__ void series_step2(double e0, double e1, double g0, do
     }
 }
 
-// The density over a nuclear step: the power series for the default five sub-steps wherever it gives what they
-// give, else the sub-steps.  The choice is each trajectory's own, so results do not depend on which
-// trajectories share a wavefront.  R: the nuclear precision.
+// The density over a nuclear step: the power series for the default five sub-steps (series) wherever it gives what
+// they give, else the sub-steps.  The choice is each trajectory's own, so results do not depend on which
+// trajectories share a wavefront; one whose lanes split between the two forms pays for both, up to 19% more than
+// the sub-steps alone, which the caller avoids where it can tell beforehand.  R: the nuclear precision.
 //  * FP64 nuclei: where the difference per step stays below tol64 (over Tully's models it is 1e-13 at most; the
 //    sub-steps' own error there is up to 1e-10) and the orders leave less than 1e-16.
 //  * FP32 nuclei: up to z2 = 4, where the 20 orders leave at most 1.3e-11 and the sub-steps' own error is
-//    1e-7 to 1e-5 (a wavefront whose lanes split between the two forms pays for both).
+//    1e-7 to 1e-5.
 template <typename R>
 __device__ __forceinline__ void propagate2(const Interp2& P, Sig2& u, double t, double tc, double dt, int nsub,
-                                           double tol64 = 1e-12) {
+                                           bool series, double tol64 = 1e-12) {
     const double s0 = t - tc;
     const double e0 = dt * fma(P.dE1, s0, P.dE0), g0 = (2.0 * dt) * fma(P.w1, s0, P.w0);
     const double e1 = (dt * dt) * P.dE1, g1 = (2.0 * dt * dt) * P.w1;
     const double b = fabs(e1) + fabs(g1);
     const double z2 = fma(4.0, b, fma(e0, e0, g0 * g0));
-    bool series = nsub == 5;
     if constexpr (sizeof(R) == 8) {
         const double m = fabs(e0) + fabs(g0) + b, m2 = m * m;
         series = series && z2 < 0.99 && 1.5e-8 * (m2 * m2) * b < tol64;

@@ -183,7 +183,7 @@ __device__ __forceinline__ void rp_elec_propagate(const AT& A, const ModelRegs& 
     const double inv = nr_rcp(tn - E.tc);
     Interp2 Pi;
     Pi.dE0 = E.dEc; Pi.dE1 = (dEn - E.dEc) * inv; Pi.w0 = E.wc; Pi.w1 = (w - E.wc) * inv;
-    propagate2<R>(Pi, E.s, t, E.tc, A.dt, A.nsub);
+    propagate2<R>(Pi, E.s, t, E.tc, A.dt, A.nsub, A.nsub == 5);
     E.dEc = dEn; E.wc = w; E.tc = tn;
 }
 

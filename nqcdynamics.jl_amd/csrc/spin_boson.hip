@@ -281,7 +281,7 @@ __device__ __forceinline__ void sb_body(const SbArgs* __restrict__ Ap, SbVec<R>*
         Interp2 P;
         P.dE0 = dEc; P.dE1 = (dEn - dEc) * inv; P.w0 = wc; P.w1 = (w - wc) * inv;
         // 100 modes carry a step's difference on: held two orders tighter beside FP64 nuclei
-        propagate2<R>(P, s, t, tc, dt, nsub, 1e-14);
+        propagate2<R>(P, s, t, tc, dt, nsub, nsub == 5, 1e-14);
         dEc = dEn; wc = w; tc = tn; t = tn;
         // the save precedes the hop callback (a save time holds the state before the step's callbacks)
         if (save_every > 0 && ((step + 1) % save_every) == 0) sb_save(Ap, tid, (step + 1) / save_every, method, st, tr, s, U);
