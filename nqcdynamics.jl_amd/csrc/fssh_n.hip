@@ -4,9 +4,11 @@
 // Restates bab_electronics.jl:48-91 for n states: velocity Verlet with the active-surface force
 // (fssh.jl:67-74) or the mean-field force with the full U^T dV U (ehrenfest.jl:50-68), the n x n
 // density propagated under V(tau) = diag(E) - i (v.d) interpolated linearly between the step ends
-// (electronic_dynamics.jl:15-79,104-140) by a power series with the error of five Tsit5 sub-steps, or
-// by the sub-steps themselves where another number is asked for, then the HoppingCallback (fssh.jl:96-121,
-// surface_hopping.jl:64-168).
+// (electronic_dynamics.jl:15-79,104-140), then the HoppingCallback (fssh.jl:96-121,
+// surface_hopping.jl:64-168).  The density takes a power series for the default five sub-steps.  With FP64
+// nuclei it serves where the error of five Tsit5 sub-steps stays below 1e-12, and the sub-steps are taken
+// elsewhere; with FP32 nuclei it gives the equation's solution at every step length (in up to 64 parts), which
+// five sub-steps miss by 1e-5 at a generator norm of 3 and by 7e-4 at 6.  Other counts are sub-steps in both.
 //
 // One trajectory per lane, all of its state in registers, lanes refilled from a work queue as
 // trajectories terminate (as the two-state kernel).  The kernel is instantiated for a maximum state

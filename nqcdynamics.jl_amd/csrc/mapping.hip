@@ -161,8 +161,10 @@ __device__ __forceinline__ void map_electronic_step(const LaneN<NM, double>& L, 
     }
 }
 
-// Bound by vector issue (Jacobi sweeps, a sincos a state).  At three states 16 registers fewer than the compiler would
-// take fit a third wavefront a SIMD (12 bytes of scratch): 5e5 trajectories x 500 steps 11.9 -> 11.5 ms.
+// Bound by vector issue (Jacobi sweeps, a sincos a state).  Three states fit a third wavefront a SIMD at 168 registers
+// instead of 178, with 12 bytes of scratch: 10.05 -> 9.64 ms for 5e5 trajectories x 500 steps, and 3 to 4% the other way
+// where the chip is not full (2.49 -> 2.57 ms for 1e5, 1.42 -> 1.49 for 2e4).  Four states take 276 and one wavefront; held
+// to two (72 bytes of scratch) they measure 23.3 -> 21.8, 5.96 -> 5.52 and 2.88 -> 3.01 ms, left for the small ensembles.
 template <int NM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NM == 3 ? 3 : 1))) void mapping_kernel(const MapArgs A) {
     const int64_t nt = A.ntraj;

@@ -140,9 +140,10 @@ __device__ __forceinline__ bf16x8 pack8(const float* lo, const float* hi) {
 // fragment read.  G is that of sample gj (this lane's own, j, unless the caller wants another's).  Optional outputs for training: h1, s1 = 1 - h1^2,
 // h2, s2 of this lane's units.
 //
-// A tile with gradients takes 160 MFMA (2800 cycles) and about 820 vector instructions, 128 of them transcendental
-// (4800 cycles), so the vector unit bounds it.  One factor per tanh and the
-// gradient fetched once per owner: 224 -> 216 ms for 2e5 trajectories of up to 3000 steps.
+// A tile with gradients takes 160 MFMA (2800 cycles) and about 820 vector instructions, 128 of them transcendental at a
+// quarter of the rate (4800 cycles).  One wavefront's chain of layers runs them one after the other, and at two
+// wavefronts a SIMD they hardly overlap: 70 and 141 ms make up 211 of the 213 ms of 2e5 trajectories of up to 3000
+// steps.  One factor per tanh and the gradient fetched once per owner: 224 -> 216 ms.
 template <bool kGrad>
 __device__ __forceinline__ void mlp_tile(const unsigned char* __restrict__ W, const float xs[kMlpIn], float o[kMlpOut],
                                          float G[kMlpOut][kMlpIn], int gj = __lane_id() & 15, float* h1_out = nullptr,

@@ -108,9 +108,10 @@ __device__ __forceinline__ SbTab<R> sb_here(SbTab<R> p) {
 // The positions of the last NL modes stay in LDS ([chunk][lane], 16 bytes a lane and access), the rest and all
 // velocities in registers: with all 2 NB values in registers a wavefront took 352 registers, so the 1,563
 // wavefronts of 1e5 trajectories ran one to a SIMD in two rounds; with 48 of the FP32 positions in LDS two fit.
-// Bound by FP32 and FP64 issue (a step is about 600 FP32 instructions for the bath and 450 for the electronics).
-// 1e5 FSSH trajectories x 1000 steps: 23.7 -> 9.2 ms; before, the coefficients were vector loads through the
-// argument pointer, each waited for, 25 round trips to the cache per pass.
+// Bound by FP32 and FP64 issue: 2,240 vector instructions a wavefront-step by the counters (700 for the bath, about 450
+// for the electronics, the hop's pass in nearly every step, as a lane hops in every sixteenth), 7.5 ms where two
+// wavefronts share a SIMD.  1e5 FSSH trajectories x 1000 steps: 23.7 -> 9.3 ms; before, the coefficients were vector
+// loads through the argument pointer, each waited for, 25 round trips to the cache per pass.
 template <int NB, int NL, typename R>
 __device__ __forceinline__ void sb_body(const SbArgs* __restrict__ Ap, SbVec<R>* lds) {
     static_assert(NB % 4 == 0 && NL % 4 == 0 && NL < NB, "chunks of four modes");
