@@ -145,7 +145,8 @@ typedef struct {
     int32_t rescaling;           /* enum nqcd_rescaling */
     int32_t precision;           /* enum nqcd_precision */
     int32_t schedule;            /* enum nqcd_schedule */
-    int32_t electronic_substeps; /* Tsit5 sub-steps per nuclear step; 0 -> 5 (bab_electronics.jl:42) */
+    int32_t electronic_substeps; /* Tsit5 sub-steps per nuclear step; 0 -> 5 (bab_electronics.jl:42), which a power series
+                                  * may stand in for (three states and more with FP32 nuclei: without their error) */
     int32_t decoherence;         /* IESH: enum nqcd_decoherence */
     const double* masses;        /* natoms (simulations.jl:86-91) */
     double dt;                   /* nuclear time step (run_dynamics.jl:71-73 default 1.0) */

@@ -339,12 +339,13 @@ __device__ __forceinline__ int ie_tid() {
 }
 #define IE_IDS const int tid = ie_tid(), w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63; (void)w; (void)l;
 
-// Bound by the matrix cores in the propagator (8 or 9 terms of N x N x 2 Ne; 109 of a step's 140 us at 101 states, where
-// seven wavefronts share four SIMDs) and, up to 64 states, by the latency of the phases around it, which one workgroup
-// cannot hide: there the registers are held to three wavefronts a SIMD, so that three or four trajectories share a
-// compute unit.  Larger problems fill the LDS with one trajectory and keep two wavefronts' registers.  The phases
-// exchange sums once (coupling norm, hop bound, orbital weight ride on the propagator's registers and barriers),
-// divide by Newton-Raphson reciprocals, save populations by a product on the matrix cores and invert S in registers.
+// Bound by the propagator (8 or 9 terms of N x N x 2 Ne on FP64 MFMA, two barriers and an LDS round trip a term: the
+// matrix cores are busy for 17.7 of 55 ms at 41 states and 29.4 of 66 ms at 101, where seven wavefronts share four
+// SIMDs) and, up to 64 states, by the latency of the phases around it, which one workgroup cannot hide: there the
+// registers are held to three wavefronts a SIMD, so that three or four trajectories share a compute unit.  Larger
+// problems fill the LDS with one trajectory and keep two wavefronts' registers.  The phases exchange sums once
+// (coupling norm, hop bound, orbital weight ride on the propagator's registers and barriers), divide by Newton-Raphson
+// reciprocals, save populations by a product on the matrix cores and invert S in registers.
 // 8192 trajectories of 41 states, 100 steps: 91 -> 56 ms; 2048 of 101 states, 50 steps: 103 -> 66 ms.
 // RPB: ring polymer (BCBWavefunction), a separate instantiation so the one-bead kernels carry none of it
 template <int NT, int CTM, bool RPB>
